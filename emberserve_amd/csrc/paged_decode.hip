@@ -17,17 +17,24 @@
 // walks every 4th 32-key tile of the split's range with its own online-softmax state, and
 // the waves merge through LDS at the end. Per tile (32 keys, v_mfma_f32_16x16x32):
 //   S^T[16 keys, 16 heads] = K[16 keys, D] . Q^T[D, 16 heads]       (2 halves x D/32 MFMAs)
-//     A = K: lane (n, g) holds key row n, d = 32c + 8g + [0, 8) for MFMA c, so one
-//            dwordx4 load instruction covers 64 contiguous bytes of 16 key rows;
+//     A = K: lane (n, g) holds key row n, d = 32c + 8g + [0, 8) for MFMA c, read back from
+//            the wave's LDS tile;
 //     B = Q^T: lane (n, g) holds head n at the same d (zero for padded heads);
 //     C: lane (n, g) gets head n's scores for keys 16s + 4g + i, i < 4.
 //   O^T[16 d, 16 heads] += V^T[16 d, 32 kslots] . P^T[32 kslots, 16 heads]   (D/16 MFMAs)
 //     kslot 8g + 4s + i <-> key 16s + 4g + i, so B = P^T is exactly the lane's own 8
 //     probabilities (head n) in register order; A = V^T needs 8 keys of one d per lane,
-//     which a wave-private LDS tile Vt[d][kslot] provides (V goes in as 2-byte scatters,
-//     comes out as one 16-byte read per d tile);
+//     which the transpose reads of the wave's LDS tile provide;
 //     C: lane (n, g) accumulates O[head n, 16 dt + 4g + i]: the head is the lane's own, so
 //     the online-softmax rescale needs no cross-lane traffic.
+//   K, then V, of a tile pass through one wave-private LDS tile in row order, so the loads
+//   from HBM need no operand layout: an instruction covers whole rows (4 of 256 bytes at
+//   D = 128, 8 of 128 at D = 64). What bounds the kernel is the K/V stream. Loads in the
+//   operand's layout (64 bytes of 16 rows per instruction) kept a CU's address path busy
+//   and needed the cache to merge the halves of a line. Measured (bf16, GPU time): 64 x
+//   4096 keys, 32q/8kv x 128: 198.5 -> 175.4 us (5.4 -> 6.1 TB/s); 64 ragged contexts up
+//   to 8192: 235.7 -> 199.7; 128 x 2048 at 14q/2kv x 64: 27.7 -> 23.9; of these, whole rows
+//   alone gave 193.0, 216.5 and 27.3, non-temporal loads the rest.
 //   The row max of a head is over its 4 lane groups (two xor shuffles per tile); the row
 //   sum stays per lane until the end.
 //
@@ -96,17 +103,11 @@ struct DecodeArgs {
   uint32_t* err;
 };
 
-#ifndef EMBER_DECODE_NT
-#define EMBER_DECODE_NT 0
-#endif
-
-// K/V loads. Measured on MI355X (128 x 2048 keys, 8 KV heads, D=128): ordinary loads
-// 5.4 TB/s, streaming (nt) loads 4.9 TB/s: the four dwordx4 instructions that cover one
-// key row's 128-byte lines merge in the cache only when the lines are allocated.
+// K/V loads: streaming (non-temporal), every byte is read once per KV head and an
+// instruction covers whole 128-byte lines.
 template <typename T>
 __device__ __forceinline__ Pack<T, 8> load_kv(const T* p) {
-  if constexpr (EMBER_DECODE_NT) return load_stream<T, 8>(p);
-  else return load_pack<T, 8>(p);
+  return load_stream<T, 8>(p);
 }
 
 // s_waitcnt immediate for vmcnt(0) with expcnt and lgkmcnt left unconstrained (gfx9
@@ -189,9 +190,12 @@ __global__ void __launch_bounds__(NW * kWave)
 k_decode_mfma(DecodeArgs a) {
   using M = Mfma<T>;
   using V8 = typename M::v8;
-  constexpr int NP = D / 32;       // 16-byte packs per lane per key row (= QK MFMAs per half)
+  constexpr int NP = D / 32;       // QK MFMAs per 16-key half tile
   constexpr int NDT = D / 16;      // d tiles of P.V
-  constexpr int VS = D + kVtPad;   // LDS row stride of the V tile (elements)
+  constexpr int VS = D + kVtPad;   // LDS row stride of the wave's tile (elements)
+  constexpr int LPR = D / 8;       // lanes per key row of a load (whole rows)
+  constexpr int RPI = kWave / LPR; // key rows per load instruction
+  constexpr int NI = 16 / RPI;     // load instructions per 16-key half tile, K and V each
   constexpr int CH = KT * NW;      // tiles between two chunks of one wave
   struct Combine {
     float m[NW][16];
@@ -239,10 +243,12 @@ k_decode_mfma(DecodeArgs a) {
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // The wave's V tiles: KT * 32 key rows (relative key order), row stride VS.
+  // The wave's tiles: KT * 32 key rows (relative key order) of K, then of V, row stride VS.
   T* vl = reinterpret_cast<T*>(lds) + w * (KT * kTile * VS);
-  const T* kbase = static_cast<const T*>(a.kc) + kvh * a.k_sh + 8 * g;
-  const T* vbase = static_cast<const T*>(a.vc) + kvh * a.v_sh + 8 * g;
+  const int lr = lane / LPR;            // this lane's row of an instruction's RPI rows
+  const int lc = (lane % LPR) * 8;      // and its d
+  const T* kbase = static_cast<const T*>(a.kc) + kvh * a.k_sh + lr * a.k_sslot + lc;
+  const T* vbase = static_cast<const T*>(a.vc) + kvh * a.v_sh + lr * a.v_sslot + lc;
   const int32_t* btrow = a.bt + b * a.bt_sb;
   // ds_read_b64_tr_b16 gives lane 4a+e of a 16-lane group element e of the 8 bytes that
   // lanes a, a+4, a+8, a+12 address. Lane n (a = n%4, jj = n/4) of group g therefore
@@ -270,8 +276,8 @@ k_decode_mfma(DecodeArgs a) {
   // Loads of the wave's chunk k (KT tiles from tile tc): a half past the context still
   // loads (from the last valid half's block) so the loads stay unconditional; keys past the
   // split's range are masked after the scores.
-  Pack<T, 8> kr[KT][2][NP];
-  Pack<T, 8> vr[KT][2][NP];
+  Pack<T, 8> kr[KT][2][NI];
+  Pack<T, 8> vr[KT][2][NI];
   auto load_chunk = [&](int tc, int k) {
 #pragma unroll
     for (int u = 0; u < KT; ++u)
@@ -281,13 +287,13 @@ k_decode_mfma(DecodeArgs a) {
         if (hk0 >= ctx) hk0 = (ctx - 1) & ~15;
         const int lb = static_cast<int>(a.bdiv.div(static_cast<uint32_t>(hk0)));
         const int pb = __builtin_amdgcn_readlane(blk_win, (((k % WIN) * KT + u) << 1) | s);
-        const int slot = hk0 - lb * a.block_size + n;
+        const int slot = hk0 - lb * a.block_size;
         const T* kp = kbase + pb * a.k_sblk + slot * a.k_sslot;
         const T* vp = vbase + pb * a.v_sblk + slot * a.v_sslot;
 #pragma unroll
-        for (int c = 0; c < NP; ++c) kr[u][s][c] = load_kv<T>(kp + 32 * c);
+        for (int c = 0; c < NI; ++c) kr[u][s][c] = load_kv<T>(kp + RPI * c * a.k_sslot);
 #pragma unroll
-        for (int c = 0; c < NP; ++c) vr[u][s][c] = load_kv<T>(vp + 32 * c);
+        for (int c = 0; c < NI; ++c) vr[u][s][c] = load_kv<T>(vp + RPI * c * a.v_sslot);
       }
   };
 
@@ -305,7 +311,15 @@ k_decode_mfma(DecodeArgs a) {
     const int k0 = tc * kTile;
     const bool partial = k0 + KT * kTile > kend;  // wave-uniform
 
-    // scores
+    // K rows into the wave's tiles, back as MFMA operands for the scores
+#pragma unroll
+    for (int u = 0; u < KT; ++u)
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int c = 0; c < NI; ++c)
+          store_pack<T, 8>(vl + (kTile * u + 16 * s + RPI * c + lr) * VS + lc, kr[u][s][c]);
+    asm volatile("" ::: "memory");
     f32x4 sc[KT][2];
 #pragma unroll
     for (int u = 0; u < KT; ++u)
@@ -313,26 +327,30 @@ k_decode_mfma(DecodeArgs a) {
       for (int s = 0; s < 2; ++s) {
         sc[u][s] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int c = 0; c < NP; ++c) sc[u][s] = M::run(__builtin_bit_cast(V8, kr[u][s][c]), qv[c], sc[u][s]);
+        for (int c = 0; c < NP; ++c) {
+          const V8 kf = *reinterpret_cast<const V8*>(vl + (kTile * u + 16 * s + n) * VS + 32 * c + 8 * g);
+          sc[u][s] = M::run(kf, qv[c], sc[u][s]);
+        }
       }
-    // V rows into the wave's tiles; rows past the split's range are stored as zero so that
-    // stale cache contents cannot turn 0 * v into NaN.
+    asm volatile("" ::: "memory");
+    // V rows into the same tiles (a wave's LDS accesses run in order); rows past the split's
+    // range are stored as zero so that stale cache contents cannot turn 0 * v into NaN.
     if (partial) {
 #pragma unroll
       for (int u = 0; u < KT; ++u)
 #pragma unroll
         for (int s = 0; s < 2; ++s)
-          if (k0 + kTile * u + 16 * s + n >= kend)
 #pragma unroll
-            for (int c = 0; c < NP; ++c) vr[u][s][c] = Pack<T, 8>{};
+          for (int c = 0; c < NI; ++c)
+            if (k0 + kTile * u + 16 * s + RPI * c + lr >= kend) vr[u][s][c] = Pack<T, 8>{};
     }
 #pragma unroll
     for (int u = 0; u < KT; ++u)
 #pragma unroll
       for (int s = 0; s < 2; ++s)
 #pragma unroll
-        for (int c = 0; c < NP; ++c)
-          store_pack<T, 8>(vl + (kTile * u + 16 * s + n) * VS + 32 * c + 8 * g, vr[u][s][c]);
+        for (int c = 0; c < NI; ++c)
+          store_pack<T, 8>(vl + (kTile * u + 16 * s + RPI * c + lr) * VS + lc, vr[u][s][c]);
     asm volatile("" ::: "memory");
     // K and V of this chunk are consumed (scores issued, V in LDS): the registers take the
     // wave's next chunk while this one's softmax and P.V run.

@@ -215,6 +215,31 @@ def test_decode_long_contexts_cross_block_id_windows(hq, hkv, d, dtype, block):
     assert _lib.read_errors() == 0
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (32, 8, 128)])
+def test_decode_strided_caches_and_stale_rows(dtype, hq, hkv, d):
+    """The key rows' load map at its edges: contexts around the rows of one load instruction
+    (4 or 8), a half tile, a tile and a round of all waves; K in a head-major cache and V in a
+    padded one (other slot, head and block strides than the packed layout's); every slot past
+    a context holds NaN, which may reach no result."""
+    ctx = [1, 3, 4, 5, 8, 9, 15, 16, 17, 31, 32, 33, 127, 128, 129, 257]
+    q, kc, vc, bt, cl = gen.decode_inputs(ctx, hq, hkv, d, 16, dtype, seed=90 + d)
+    dq, dbt, dcl = _to_dev(q, bt, cl)
+    live = torch.zeros(kc.shape[:2], dtype=torch.bool)
+    for b, n in enumerate(ctx):
+        for j in range(n):
+            live[bt[b, j // 16], j % 16] = True
+    k_dev = torch.full((kc.shape[0], hkv, 16, d), float("nan"), dtype=dtype, device=DEV).transpose(1, 2)
+    v_dev = torch.full((kc.shape[0], 16, hkv, d + 8), float("nan"), dtype=dtype, device=DEV)[..., :d]
+    k_dev[live.to(DEV)] = kc[live].to(DEV)
+    v_dev[live.to(DEV)] = vc[live].to(DEV)
+    want = _want(q, kc, vc, bt, cl, d ** -0.5)
+    for splits in (1, 3):
+        got = paged_attention_decode(dq, k_dev, v_dev, dbt, dcl, d ** -0.5, num_splits=splits)
+        _check(got, q, kc, vc, bt, cl, d ** -0.5, True, f"{hq}/{hkv}/{d} splits={splits}", want)
+    assert _lib.read_errors() == 0
+
+
 def test_decode_full_size_split_invariance_and_sampled_parity():
     """The bench size (128 sequences x 2048 keys, 14q/2kv D=64 fp16, block 16): the default
     split and one split agree within the split-K rounding; four sampled sequences are
