@@ -96,6 +96,7 @@ struct DecodeArgs {
   int32_t d;
   float scale2;                // scale * log2(e)
   int32_t splits;
+  int32_t min_tiles;           // MFMA kernel: the least tiles a split takes
   float* part_m;               // [splits][nseq][nh]
   float* part_l;
   float* part_o;               // [splits][nseq][nh][d]
@@ -146,14 +147,28 @@ __device__ __forceinline__ int phys_block(const DecodeArgs& a, const int32_t* bt
   return p;
 }
 
-// Key-tile range [t0, t1) of split `split` (tiles of kTile keys), as every kernel here
-// partitions it: the real context, not the table width, is split.
+// Key-tile range [t0, t1) of split `split` (tiles of kTile keys) in the fp32 kernel: the
+// real context, not the table width, is split.
 __device__ __forceinline__ void split_range(int ctx, int splits, int split, int& t0, int& t1) {
   const int nt = (ctx + kTile - 1) / kTile;
   const int per = (nt + splits - 1) / splits;
   t0 = split * per;
   t1 = min(t0 + per, nt);
 }
+
+// Tiles per split of the MFMA kernel: the context in equal parts, but no part under min_tiles,
+// so a short context of a ragged batch takes fewer splits than a long one (at least one).
+__device__ __forceinline__ int tiles_per_split(const DecodeArgs& a, int nt) {
+  return max((nt + a.splits - 1) / a.splits, a.min_tiles);
+}
+
+// The least tiles per split on a full grid (more than kFullGridPerCu workgroups per CU):
+// there a split's fixed cost (context, block ids and first rows in turn, its share of the
+// merge: ~5 us) is paid out of bandwidth others could use, so parts stay >= 512 keys. A
+// small grid splits as asked: its CUs would idle otherwise (B = 1 x 8192, 32q/8kv x 128, 16
+// splits: 11.9 us without a least, 13.4 at 512 keys).
+constexpr int kFullGridTiles = 16;
+constexpr int kFullGridPerCu = 2;
 
 // Tiles per loop iteration (KT) and next-iteration prefetch (PF) per head dim. Measured on
 // MI355X: prefetch lifts D=128 from 5.35 to 5.6 TB/s (128 x 2048 keys, 8 KV heads).
@@ -211,18 +226,43 @@ k_decode_mfma(DecodeArgs a) {
   const int n = lane & 15;
   const int g = lane >> 4;
 
-  int pid = blockIdx.x;
-  const int hc = pid % a.hchunks;
-  pid /= a.hchunks;
-  const int kvh = pid % a.nkv;
-  const int b = pid / a.nkv;
-  const int split = blockIdx.y;
+  // Workgroup order: units (sequence, split), eight at a time, one per XCD (the dispatcher
+  // gives workgroup i to XCD i % 8), and a unit's KV heads one after another on its XCD, whose
+  // rows lie side by side in the cache. The units of a group of eight are rotated by the
+  // group's number, so that split 0 (the one a short context has) does not always land on
+  // the same XCD. 64 ragged contexts up to 8192, 32q/8kv x 128, 8 splits of >= 512 keys:
+  // 191 us with one KV head per XCD, 185 in this order.
+  int u, hk;
+  {
+    const int pid = blockIdx.x + gridDim.x * blockIdx.y;
+    const int heads = a.nkv * a.hchunks;
+    const int units8 = (a.nseq * a.splits) & ~7;
+    if (pid < units8 * heads) {
+      const int grp8 = pid / (8 * heads);
+      const int r = pid - grp8 * 8 * heads;
+      u = 8 * grp8 + ((r + 7 * grp8) & 7);
+      hk = r >> 3;
+    } else {  // the last, incomplete group
+      const int rem = a.nseq * a.splits - units8;
+      const int r = pid - units8 * heads;
+      u = units8 + r % rem;
+      hk = r / rem;
+    }
+  }
+  const int hc = hk % a.hchunks;
+  const int kvh = hk / a.hchunks;
+  const int split = u % a.splits;
+  const int b = u / a.splits;
   const int head0 = kvh * a.grp + hc * 16;
   const int nhc = min(16, a.grp - hc * 16);
 
   const int ctx = seq_context(a, b);
-  int t0, t1;
-  split_range(ctx, a.splits, split, t0, t1);
+  const int nt = (ctx + kTile - 1) / kTile;
+  const int per = tiles_per_split(a, nt);
+  const int nsplit = max(1, (nt + per - 1) / per);  // splits that this context takes
+  if (split >= nsplit) return;
+  const int t0 = split * per;
+  const int t1 = min(t0 + per, nt);
   const int kend = min(t1 * kTile, ctx);  // keys of this split: [t0 * kTile, kend)
 
   // Q^T operand: head n of this chunk, d = 32c + 8g + [0, 8).
@@ -473,7 +513,7 @@ k_decode_mfma(DecodeArgs a) {
       store_pack<T, VEC>(orow + VEC * PARTS * j, r);
     }
   };
-  if (a.splits == 1) {
+  if (nsplit == 1) {
     if (mine) store_out(L);
     return;
   }
@@ -504,7 +544,7 @@ k_decode_mfma(DecodeArgs a) {
   if (threadIdx.x == 0) {
     uint32_t* cnt = a.counters + row0;
     const uint32_t prev = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    is_last = prev == static_cast<uint32_t>(a.splits - 1);
+    is_last = prev == static_cast<uint32_t>(nsplit - 1);
     if (is_last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
@@ -524,8 +564,8 @@ k_decode_mfma(DecodeArgs a) {
   float gl = 0.f;
 #pragma unroll
   for (int j = 0; j < NJ; ++j) acc[j] = FV{};
-  for (int c0 = 0; c0 < a.splits; c0 += kMergeChunk) {
-    const int cn = min(kMergeChunk, a.splits - c0);
+  for (int c0 = 0; c0 < nsplit; c0 += kMergeChunk) {
+    const int cn = min(kMergeChunk, nsplit - c0);
     float ms[kMergeChunk], ls[kMergeChunk];
     FV v[kMergeChunk][NJ];
 #pragma unroll
@@ -828,7 +868,8 @@ int paged_decode_core(const void* q, int64_t q_seq_stride, int64_t q_head_stride
   int rc = EMBER_OK;
   const bool mfma = same && dok && aligned;
   if (mfma) {
-    if (progs > INT32_MAX) return EMBER_EINVAL;
+    if (progs * num_splits > INT32_MAX) return EMBER_EINVAL;
+    a.min_tiles = progs * num_splits > kFullGridPerCu * int64_t(ncu) ? kFullGridTiles : 1;
     dim3 grid(static_cast<uint32_t>(progs), static_cast<uint32_t>(num_splits));
     rc = q_dtype == EMBER_F16 ? launch_mfma<_Float16>(a.d, nw, a, grid, st)
                               : launch_mfma<__bf16>(a.d, nw, a, grid, st);

@@ -36,6 +36,7 @@ MAX_SPLITS = 32
 TILE = 32                 # keys per kernel tile
 MIN_KEYS_PER_SPLIT = 256
 LONG_SPLIT_KEYS = 512     # keys per split at which MAX_SPLITS splits are allowed
+RAGGED_SPLIT_KEYS = 768   # keys of the table width per split on grids that fill the chip
 
 
 def interpreter_enabled() -> bool:
@@ -78,15 +79,22 @@ def default_num_splits(batch: int, num_kv_heads: int, max_context: int, device: 
     workgroup (8 waves at head_dim 64, 4 at 128) keeps one CU's share of HBM bandwidth in
     flight, and more workgroups only add merge work (measured on MI355X, rotated inputs:
     128 x 2048 keys at D=64 4.8 TB/s unsplit vs 4.4 at 2 splits; 8 x 8192 keys at D=128
-    5.0 TB/s at 4 splits = 256 workgroups). Contexts are cut into round(CUs / programs)
+    5.0 TB/s at 4 splits = 256 workgroups). At head_dim 128, grids of half a program to four
+    programs per compute unit are cut finer, to RAGGED_SPLIT_KEYS keys of the table width: the
+    contexts of a batch differ, and one workgroup per (sequence, KV head) leaves the CUs that
+    got the longest running alone at the end. Measured (contexts uniform in [1, width], bf16,
+    us at the splits of one program per CU | at this rule's): 32q/8kv, 64 x 8192 213 | 188,
+    64 x 4096 111 | 99, 32 x 8192 116 | 100, 16 x 4096 33.6 | 31.5; 28q/4kv, 40 x 3008 36.8 |
+    35.0; at full, equal contexts it costs 5% (64 x 4096 175 | 184). From four programs per
+    CU the dispatcher balances them (128 x 2048: 109 | 105), and at head_dim 64, where a
+    workgroup has eight waves, the finer cut lost (128 x 4096 31.2 | 33.2). Contexts are cut into round(CUs / programs)
     pieces, never below MIN_KEYS_PER_SPLIT keys each, and at most MAX_SPLITS / 2 unless the
     context gives every one of MAX_SPLITS splits LONG_SPLIT_KEYS keys. `head_dim` is
-    accepted for callers that size by it; the rule does not need it.
+    the cache's (64 or 128).
     """
     forced = os.environ.get("EMBERSERVE_TRITON_SPLITS")
     if forced:
         return max(1, int(forced))
-    del head_dim
     chunks = 1
     if num_heads is not None and num_kv_heads > 0:
         chunks = -(-(num_heads // num_kv_heads) // 16)
@@ -99,7 +107,10 @@ def default_num_splits(batch: int, num_kv_heads: int, max_context: int, device: 
     # 17.4 us; ctx 16384 25.0 / 22.9; ctx 32768 41.7 / 33.5; 40-64 splits were slower than
     # 32 up to 65536 keys).
     cap = MAX_SPLITS if max_context >= MAX_SPLITS * LONG_SPLIT_KEYS else MAX_SPLITS // 2
-    return max(1, min(cap, want, by_context))
+    splits = min(cap, want, by_context)
+    if head_dim == 128 and target <= 2 * programs < 8 * target:
+        splits = max(splits, min(MAX_SPLITS // 2, max_context // RAGGED_SPLIT_KEYS))
+    return max(1, splits)
 
 
 def default_variant() -> str:

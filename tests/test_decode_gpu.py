@@ -240,6 +240,28 @@ def test_decode_strided_caches_and_stale_rows(dtype, hq, hkv, d):
     assert _lib.read_errors() == 0
 
 
+@pytest.mark.parametrize("batch,hq,hkv,d,splits", [(67, 16, 8, 128, 4), (131, 6, 3, 64, 3), (43, 40, 2, 128, 16)])
+def test_decode_ragged_batches_take_fewer_splits_for_short_contexts(batch, hq, hkv, d, splits):
+    """Full grids (more than two workgroups per CU): no split under 512 keys, so contexts up
+    to 512 keys have one split, 513 two; (sequence, split) counts that are no multiple of 8
+    (the workgroup order's last group), an empty context in the middle. Three calls on one
+    workspace: the arrival counters return to zero whatever number of splits took part."""
+    ctx = _ragged(batch, 1700, 16, seed=batch)
+    ctx[3:9] = [511, 512, 513, 1024, 1025, 0]
+    q, kc, vc, bt, cl = gen.decode_inputs(ctx, hq, hkv, d, 16, torch.bfloat16, seed=60 + batch)
+    dq, dkc, dvc, dbt, dcl = _to_dev(q, kc, vc, bt, cl)
+    rows = [b for b in range(batch) if ctx[b]]
+    want = _want(q[rows], kc, vc, bt[rows], cl[rows], d ** -0.5)
+    first = None
+    for _ in range(3):
+        got = paged_attention_decode(dq, dkc, dvc, dbt, dcl, d ** -0.5, num_splits=splits)
+        _check(got[rows], q[rows], kc, vc, bt[rows], cl[rows], d ** -0.5, True, f"B={batch}", want)
+        assert bool(torch.isnan(got[8]).all())
+        first = got if first is None else first
+        assert torch.equal(got[rows], first[rows])
+    assert _lib.read_errors() == 0
+
+
 def test_decode_full_size_split_invariance_and_sampled_parity():
     """The bench size (128 sequences x 2048 keys, 14q/2kv D=64 fp16, block 16): the default
     split and one split agree within the split-K rounding; four sampled sequences are
