@@ -19,17 +19,23 @@
 // (v_mfma_f32_16x16x32):
 //   S^T[16 keys, 16 heads] = R[16 keys, 576] . Q^T[576, 16 heads], each wave over its 9
 //   chunks (2 halves x 9 MFMAs), the two partial sums exchanged through LDS:
-//     A = R: lane (n, g) holds cache row n at e = chunk + 8g + [0, 8) (one dwordx4 load);
+//     A = R: lane (n, g) holds cache row n at e = chunk + 8g + [0, 8);
 //     B = Q^T: lane (n, g) holds head n at the same e (registers, loaded once);
 //     C: lane (n, g) gets head n's scores for keys 16s + 4g + i, i < 4.
 //   O^T[16 d, 16 heads] += C^T[16 d, 32 kslots] . P^T[32 kslots, 16 heads], over the wave's
-//   own d half (16 MFMAs): its value chunks, already in registers, go to a wave-private
-//   LDS tile as they are (row-major, 16-byte stores) and come back transposed by
-//   ds_read_b64_tr_b16, so the cache is read once; kslot 8g + 4s + i <-> key 16s + 4g + i,
-//   so P^T is the lane's own 8 probabilities; C: lane (n, g) accumulates O[head n,
-//   d0 + 16 dt + 4g + i].
-//   The next tile's rows are requested as soon as this tile's scores and values are out of
-//   the registers; block ids come from a per-pair window of 32 tiles read ahead.
+//   own d half (16 MFMAs). kslot 8g + 4s + i <-> key 16s + 4g + i, so P^T is the lane's own
+//   8 probabilities; C: lane (n, g) accumulates O[head n, d0 + 16 dt + 4g + i].
+//   A wave's half of the value part passes through a wave-private LDS tile in row order and
+//   feeds both products from there: the score operands row by row, the P.V operands through
+//   the transpose reads of ds_read_b64_tr_b16. So the loads from HBM need no operand layout:
+//   an instruction covers two 512-byte half rows, streamed past the cache when no other head
+//   chunk reads them. What bounds full grids is that stream: in the operand's layout (64
+//   bytes of 16 rows per instruction, cached) a CU's address path was busy and the cache had
+//   to merge half lines. Measured (bf16, 16 heads): 256 x 2048 keys 113 -> 95 us (5.3 -> 6.4
+//   TB/s), 256 ragged contexts up to 4096 157 -> 131, 128 up to 2048 51 -> 44, 32 x 4096 at 8
+//   splits 38 -> 34. Cached whole rows: 113, 143, 47 and 38.
+//   The next tile's rows are requested as soon as this tile's are in LDS; block ids come
+//   from a per-pair window of 32 tiles read ahead.
 //   Online softmax in base 2 with a lazy rescale: a head's reference max moves only when a
 //   tile's max exceeds it by more than kLazy (probabilities stay <= 2^kLazy, far inside
 //   fp16/bf16/fp32 range), so the accumulator rescale runs a few times per split instead of
@@ -43,7 +49,7 @@
 //
 // With num_splits > 1 the partial (m, l, acc) of each split goes to the workspace; the MFMA
 // kernel's last split to finish merges them (an arrival counter per sequence and head
-// chunk), k_mla_reduce does it for the fp32 kernel (paged_triton.py:188-209 semantics).
+// chunk), or k_mla_merge does (from 4 splits), k_mla_reduce does it for the fp32 kernel (paged_triton.py:188-209 semantics).
 //
 // Bad inputs never fault: a context length outside [0, max_blocks * block_size] is clamped
 // (EMBER_ERR_DECODE_CTX); a block id outside [0, num_blocks) reads block 0
@@ -77,7 +83,11 @@ constexpr int kTile = 32;      // keys per tile (one P.V MFMA deep)
 constexpr int kVPad = 8;       // elements of padding per LDS value row (keeps 16-byte alignment)
 constexpr float kLazy = 8.f;   // log2 headroom before the running max moves
 constexpr int kMlaPairs = 2;       // tile streams (wave pairs) per workgroup
-constexpr int kMlaPairsSmall = 4;  // ... when the grid fills at most half of the CUs
+constexpr int kMlaPairsSmall = 4;  // ... when the grid has at most one workgroup per CU
+// The least tiles per split on grids over half the CUs: 128 keys, two rounds of the tile
+// streams (32 ragged contexts up to 4096 at 24 splits 35.1 -> 32.3 us, 100 up to 512 at 4
+// splits 22.4 -> 21.8).
+constexpr int kMlaMinTiles = 4;
 #ifndef EMBER_MLA_PAIR_SYNC
 #define EMBER_MLA_PAIR_SYNC 1
 #endif
@@ -115,6 +125,7 @@ struct MlaArgs {
   int32_t dl, dr;
   float scale2;                // scale * log2(e)
   int32_t splits;
+  int32_t min_tiles;           // MFMA kernels: the least tiles a split takes
   float* part_m;               // [splits][nseq][nh]
   float* part_l;
   float* part_o;               // [splits][nseq][nh][dl]
@@ -179,14 +190,50 @@ __device__ __forceinline__ void split_range(int ctx, int splits, int split, int&
   t1 = min(t0 + per, nt);
 }
 
+// How the MFMA kernels cut a context: equal parts of at least min_tiles tiles, so a short
+// context of a ragged batch takes fewer splits than a long one (at least one).
+struct SplitPlan {
+  int per;  // tiles per split
+  int n;    // splits that the context takes
+};
+__device__ __forceinline__ SplitPlan split_plan(const MlaArgs& a, int ctx) {
+  const int nt = (ctx + kTile - 1) / kTile;
+  const int per = max((nt + a.splits - 1) / a.splits, a.min_tiles);
+  return {per, max(1, (nt + per - 1) / per)};
+}
+
+// Workgroup order of the MFMA kernels: units (sequence, split), eight at a time, one per XCD
+// (the dispatcher gives workgroup i to XCD i % 8), a unit's head chunks one after another on
+// its XCD, whose L2 then holds their common rows. The units of a group of eight are rotated
+// by the group's number, so that no XCD gets one split number (or every eighth sequence)
+// alone.
+__device__ __forceinline__ void mla_unit(const MlaArgs& a, int& b, int& split, int& hc) {
+  const int pid = blockIdx.x + gridDim.x * blockIdx.y;
+  const int units8 = (a.nseq * a.splits) & ~7;
+  int u;
+  if (pid < units8 * a.hchunks) {
+    const int grp8 = pid / (8 * a.hchunks);
+    const int r = pid - grp8 * 8 * a.hchunks;
+    u = 8 * grp8 + ((r + 7 * grp8) & 7);
+    hc = r >> 3;
+  } else {  // the last, incomplete group
+    const int rem = a.nseq * a.splits - units8;
+    const int r = pid - units8 * a.hchunks;
+    u = units8 + r % rem;
+    hc = r / rem;
+  }
+  split = u % a.splits;
+  b = u / a.splits;
+}
+
 // The end of an MFMA kernel's workgroup: the tile streams merge through LDS, then either
 // the output rows are written (one split) or the split's partial is published and the last
 // split to arrive merges all of them. m, lsum and o are the wave's online-softmax state;
 // wave w of pair w / 2 holds d in [(w % 2) DL / 2, (w % 2 + 1) DL / 2).
 template <typename T, int DL, int NP>
 __device__ __forceinline__ void mla_finish(const MlaArgs& a, unsigned char* lds, float m, float lsum,
-                                           const f32x4 (&o)[DL / 32], int b, int split, int head0,
-                                           int nhc, bool poisoned = false) {
+                                           const f32x4 (&o)[DL / 32], int b, int split, int nsplit,
+                                           int head0, int nhc, bool poisoned = false) {
   constexpr int NDT = DL / 32;
   struct Combine {
     float m[NP][16];
@@ -260,7 +307,7 @@ __device__ __forceinline__ void mla_finish(const MlaArgs& a, unsigned char* lds,
       store_pack<T, 4>(orow + 4 * PARTS * j, r);
     }
   };
-  if (a.splits == 1) {
+  if (nsplit == 1) {
     if (mine) store_out(L);
     return;
   }
@@ -289,7 +336,7 @@ __device__ __forceinline__ void mla_finish(const MlaArgs& a, unsigned char* lds,
   if (threadIdx.x == 0) {
     uint32_t* cnt = a.counters + row0;
     const uint32_t prev = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    is_last = prev == static_cast<uint32_t>(a.splits - 1);
+    is_last = prev == static_cast<uint32_t>(nsplit - 1);
     if (is_last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
@@ -305,8 +352,8 @@ __device__ __forceinline__ void mla_finish(const MlaArgs& a, unsigned char* lds,
   float gl = 0.f;
 #pragma unroll
   for (int j = 0; j < NJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int c0 = 0; c0 < a.splits; c0 += kMergeChunk) {
-    const int cn = min(kMergeChunk, a.splits - c0);
+  for (int c0 = 0; c0 < nsplit; c0 += kMergeChunk) {
+    const int cn = min(kMergeChunk, nsplit - c0);
     float ms[kMergeChunk], ls[kMergeChunk];
     f32x4 v[kMergeChunk][NJ];
 #pragma unroll
@@ -352,7 +399,7 @@ __device__ __forceinline__ void poison_state(float& m, float& lsum, f32x4 (&o)[N
   for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x4{m, m, m, m};
 }
 
-template <typename T, int DL, int DR, int NP, bool PSYNC>
+template <typename T, int DL, int DR, int NP, bool PSYNC, bool NT>
 __global__ void __launch_bounds__(NP * 2 * kWave, 2)
 k_mla_mfma(MlaArgs a) {
   using M = MlaMfma<T>;
@@ -382,21 +429,26 @@ k_mla_mfma(MlaArgs a) {
   const int n = lane & 15;
   const int g = lane >> 4;
 
-  const int hc = blockIdx.x % a.hchunks;
-  const int b = blockIdx.x / a.hchunks;
-  const int split = blockIdx.y;
+  int b, split, hc;
+  mla_unit(a, b, split, hc);
   const int head0 = hc * 16;
   const int nhc = min(16, a.nh - head0);
 
   const int ctx = seq_context(a, b);
-  int t0, t1;
-  split_range(ctx, a.splits, split, t0, t1);
+  const SplitPlan plan = split_plan(a, ctx);
+  if (split >= plan.n) return;
+  const int t0 = split * plan.per;
+  const int t1 = min(t0 + plan.per, (ctx + kTile - 1) / kTile);
   const int kend = min(t1 * kTile, ctx);
 
   // Element offset of this wave's chunk j within a row: NV value chunks of its d half,
   // then NR chunks of the rope part.
   auto chunk_e = [&](int j) { return j < NV ? (hw * NV + j) * 32 : DL + (hw * NR + (j - NV)) * 32; };
 
+  constexpr int VLPR = DL / 16;         // lanes per row of a value load (the wave's half row)
+  constexpr int VRPI = kWave / VLPR;    // rows per value load
+  static_assert(VRPI * NV == 16, "value loads of a half tile");
+  const int vr = lane / VLPR, vc = lane % VLPR;
   // The pair's physical block ids, a window of 32 tiles at a time: lane 2k + s holds the
   // block of half s of the pair's k-th tile of the window, so a tile's row loads never wait
   // on a block-table read.
@@ -413,7 +465,9 @@ k_mla_mfma(MlaArgs a) {
   // Half s of the pair's k-th tile: a half past the context still loads (from the last valid
   // half's block) so the loads stay unconditional; keys past the split's range are masked
   // after the scores.
-  const T* lbase = static_cast<const T*>(a.lat) + 8 * g;
+  const T* lat = static_cast<const T*>(a.lat);
+  const T* vbase = lat + vr * a.l_sslot + hw * (DL / 2) + 8 * vc;
+  const T* rbase = lat + n * a.l_sslot + 8 * g;
   Pack<T, 8> kr[2][NC];
   auto load_tile = [&](int k) {
 #pragma unroll
@@ -422,9 +476,12 @@ k_mla_mfma(MlaArgs a) {
       if (hk0 >= ctx) hk0 = (ctx - 1) & ~15;
       const int lb = static_cast<int>(a.bdiv.div(static_cast<uint32_t>(hk0)));
       const int pb = __builtin_amdgcn_readlane(blk_win, ((k & 31) << 1) | s);
-      const T* rp = lbase + pb * a.l_sblk + (hk0 - lb * a.block_size + n) * a.l_sslot;
+      const int64_t r0 = pb * a.l_sblk + (hk0 - lb * a.block_size) * a.l_sslot;
 #pragma unroll
-      for (int j = 0; j < NC; ++j) kr[s][j] = load_pack<T, 8>(rp + chunk_e(j));
+      for (int j = 0; j < NV; ++j)
+        kr[s][j] = NT ? load_stream<T, 8>(vbase + r0 + VRPI * j * a.l_sslot) : load_pack<T, 8>(vbase + r0 + VRPI * j * a.l_sslot);
+#pragma unroll
+      for (int j = NV; j < NC; ++j) kr[s][j] = load_pack<T, 8>(rbase + r0 + chunk_e(j));
     }
   };
   if (nloc > 0) {
@@ -507,38 +564,45 @@ k_mla_mfma(MlaArgs a) {
     if (more && ((k + 1) & 31) == 0) load_window(k + 1);
     f32x4 sc[2];
     if (active) {
+      // the tile's value rows into the wave's LDS tile (rows past the range stored as zero so
+      // that stale cache contents cannot turn 0 * v into NaN); the registers take the pair's
+      // next tile while this one's scores, exchange, softmax and P.V run
+      if (partial) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int j = 0; j < NV; ++j)
+            if (k0 + 16 * s + VRPI * j + vr >= kend) kr[s][j] = Pack<T, 8>{};
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int j = 0; j < NV; ++j) store_pack<T, 8>(vl + (16 * s + VRPI * j + vr) * VS + 8 * vc, kr[s][j]);
+      Pack<T, 8> rp[2][NR];
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int j = 0; j < NR; ++j) rp[s][j] = kr[s][NV + j];
+      asm volatile("" ::: "memory");
+      if (more) load_tile(k + 1);
       // partial scores over this wave's chunks (two accumulation chains per half)
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         f32x4 c0 = f32x4{0.f, 0.f, 0.f, 0.f}, c1 = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < NC; j += 2) {
-          c0 = M::run(__builtin_bit_cast(V8, kr[s][j]), qv[j], c0);
-          if (j + 1 < NC) c1 = M::run(__builtin_bit_cast(V8, kr[s][j + 1]), qv[j + 1], c1);
+        for (int j = 0; j < NC; ++j) {
+          const V8 kf = j < NV ? *reinterpret_cast<const V8*>(vl + (16 * s + n) * VS + 32 * j + 8 * g)
+                               : __builtin_bit_cast(V8, rp[s][j - NV]);
+          if (j % 2 == 0) c0 = M::run(kf, qv[j], c0);
+          else c1 = M::run(kf, qv[j], c1);
         }
         sc[s] = c0 + c1;
       }
-      // values of this wave's d half into its LDS tile (rows past the range stored as zero
-      // so that stale cache contents cannot turn 0 * v into NaN), partial scores out
-      if (partial) {
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-          if (k0 + 16 * s + n >= kend)
-#pragma unroll
-            for (int j = 0; j < NV; ++j) kr[s][j] = Pack<T, 8>{};
-      }
-#pragma unroll
-      for (int s = 0; s < 2; ++s)
-#pragma unroll
-        for (int j = 0; j < NV; ++j) store_pack<T, 8>(vl + (16 * s + n) * VS + 32 * j + 8 * g, kr[s][j]);
       if constexpr (PSYNC) pair_wait(&sync_rd[w ^ 1], k);
       xs[(w * 2 + 0) * kWave + lane] = sc[0];
       xs[(w * 2 + 1) * kWave + lane] = sc[1];
       if constexpr (PSYNC) pair_post(&sync_wr[w], k + 1);
       asm volatile("" ::: "memory");
-      // the registers take the pair's next tile while this one's exchange, softmax and P.V
-      // run
-      if (more) load_tile(k + 1);
     }
     if constexpr (PSYNC) pair_wait(&sync_wr[w ^ 1], k + 1);
     else __syncthreads();
@@ -607,7 +671,7 @@ k_mla_mfma(MlaArgs a) {
   // the output rows of this workgroup (or the merge of its split) come out NaN instead of a
   // plausible wrong value, next to the EMBER_ERR_SYNC bit.
   if (!sync_ok) poison_state(m, lsum, o);
-  mla_finish<T, DL, NP>(a, lds, m, lsum, o, b, split, head0, nhc, !sync_ok);
+  mla_finish<T, DL, NP>(a, lds, m, lsum, o, b, split, plan.n, head0, nhc, !sync_ok);
 }
 
 // k_mla_lds: the small-grid form of k_mla_mfma (same work split: two wave pairs per
@@ -648,15 +712,16 @@ k_mla_lds(MlaArgs a) {
   const int n = lane & 15;
   const int g = lane >> 4;
 
-  const int hc = blockIdx.x % a.hchunks;
-  const int b = blockIdx.x / a.hchunks;
-  const int split = blockIdx.y;
+  int b, split, hc;
+  mla_unit(a, b, split, hc);
   const int head0 = hc * 16;
   const int nhc = min(16, a.nh - head0);
 
   const int ctx = seq_context(a, b);
-  int t0, t1;
-  split_range(ctx, a.splits, split, t0, t1);
+  const SplitPlan plan = split_plan(a, ctx);
+  if (split >= plan.n) return;
+  const int t0 = split * plan.per;
+  const int t1 = min(t0 + plan.per, (ctx + kTile - 1) / kTile);
   const int kend = min(t1 * kTile, ctx);
 
   const int32_t* btrow = a.bt + b * a.bt_sb;
@@ -862,7 +927,7 @@ k_mla_lds(MlaArgs a) {
   // the output rows of this workgroup (or the merge of its split) come out NaN instead of a
   // plausible wrong value, next to the EMBER_ERR_SYNC bit.
   if (!sync_ok) poison_state(m, lsum, o);
-  mla_finish<T, DL, NP>(a, lds, m, lsum, o, b, split, head0, nhc, !sync_ok);
+  mla_finish<T, DL, NP>(a, lds, m, lsum, o, b, split, plan.n, head0, nhc, !sync_ok);
 }
 
 constexpr int kAnyMaxD = 1024;          // DL + DR of the fp32 kernel
@@ -1007,9 +1072,13 @@ k_mla_merge(MlaArgs a) {
   if (row >= a.nseq * a.nh) return;
   const int d = (t % TPR) * 4;
   const int64_t stride = int64_t(a.nseq) * a.nh;
+  const int b = row / a.nh;
+  const int cap = a.max_blocks * a.block_size;
+  const int nsplit = split_plan(a, min(max(a.ctx[b], 0), cap)).n;
+  if (nsplit == 1) return;  // its only split wrote the output rows
   float gm = -INFINITY, gl = 0.f;
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int c0 = 0; c0 < a.splits; c0 += kChunk) {
+  for (int c0 = 0; c0 < nsplit; c0 += kChunk) {
     float ms[kChunk], ls[kChunk];
     f32x4 v[kChunk];
 #pragma unroll
@@ -1017,7 +1086,7 @@ k_mla_merge(MlaArgs a) {
       ms[u] = -INFINITY;
       ls[u] = 0.f;
       v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (c0 + u < a.splits) {
+      if (c0 + u < nsplit) {
         const int64_t r = (c0 + u) * stride + row;
         ms[u] = a.part_m[r];
         ls[u] = a.part_l[r];
@@ -1041,12 +1110,29 @@ k_mla_merge(MlaArgs a) {
     }
     gm = cm;
   }
-  const int b = row / a.nh;
   const int h = row - b * a.nh;
   Pack<TO, 4> r;
 #pragma unroll
   for (int e = 0; e < 4; ++e) r.v[e] = from_f32<TO>(acc[e] / gl);
   store_pack<TO, 4>(static_cast<TO*>(a.out) + b * a.o_sb + h * a.o_sh + d, r);
+}
+
+template <typename T, bool NT>
+void launch_register_mfma(const MlaArgs& a, dim3 grid, bool four, hipStream_t st) {
+  if (four)
+    k_mla_mfma<T, kMlaDL, kMlaDR, kMlaPairsSmall, kMlaPairSync, NT><<<grid, kMlaPairsSmall * 2 * kWave, 0, st>>>(a);
+  else
+    k_mla_mfma<T, kMlaDL, kMlaDR, kMlaPairs, kMlaPairSync, NT><<<grid, kMlaPairs * 2 * kWave, 0, st>>>(a);
+}
+
+template <typename T>
+void launch_mfma(const MlaArgs& a, dim3 grid, bool small, bool four, hipStream_t st) {
+  if (small && kMlaStaged)
+    k_mla_lds<T, kMlaDL, kMlaDR><<<grid, 4 * kWave, 0, st>>>(a);
+  else if (a.hchunks == 1)  // every row has one reader: stream it
+    launch_register_mfma<T, true>(a, grid, four, st);
+  else
+    launch_register_mfma<T, false>(a, grid, four, st);
 }
 
 template <typename TQ>
@@ -1157,28 +1243,23 @@ int ember_mla_decode(const void* q_c, int64_t qc_seq_stride, int64_t qc_head_str
   int rc = EMBER_OK;
   if (mfma) {
     const int64_t progs = num_seqs * a.hchunks;
-    if (progs > INT32_MAX) return EMBER_EINVAL;
+    if (progs * num_splits > INT32_MAX) return EMBER_EINVAL;
     dim3 grid(static_cast<uint32_t>(progs), static_cast<uint32_t>(num_splits));
     // A grid that fills at most half of the CUs (one or a few sequences) runs four tile
     // streams per workgroup: half the serial tiles per stream, one workgroup per CU.
     const int ncu = device_cu_count();
     const bool small = ncu > 0 && progs * num_splits * 2 <= ncu;
+    // Up to one workgroup per CU, four streams too once a split can hold two tiles for each:
+    // 32 ragged contexts up to 4096 at 8 splits 29.3 -> 28.8 us (equal ones 34.7 -> 33.7),
+    // but 128 x 320 keys at 2 splits 19.0 -> 19.7.
+    const bool four = small || (ncu > 0 && progs * num_splits <= ncu &&
+                                max_blocks * block_size >= num_splits * 2 * kMlaPairsSmall * kTile);
+    a.min_tiles = small ? 1 : kMlaMinTiles;
     a.merge_apart = num_splits >= kMlaMergeApart ? 1 : 0;
-    if (q_dtype == EMBER_F16) {
-      if (small && kMlaStaged)
-        k_mla_lds<_Float16, kMlaDL, kMlaDR><<<grid, 4 * kWave, 0, st>>>(a);
-      else if (small)
-        k_mla_mfma<_Float16, kMlaDL, kMlaDR, kMlaPairsSmall, kMlaPairSync><<<grid, kMlaPairsSmall * 2 * kWave, 0, st>>>(a);
-      else
-        k_mla_mfma<_Float16, kMlaDL, kMlaDR, kMlaPairs, kMlaPairSync><<<grid, kMlaPairs * 2 * kWave, 0, st>>>(a);
-    } else {
-      if (small && kMlaStaged)
-        k_mla_lds<__bf16, kMlaDL, kMlaDR><<<grid, 4 * kWave, 0, st>>>(a);
-      else if (small)
-        k_mla_mfma<__bf16, kMlaDL, kMlaDR, kMlaPairsSmall, kMlaPairSync><<<grid, kMlaPairsSmall * 2 * kWave, 0, st>>>(a);
-      else
-        k_mla_mfma<__bf16, kMlaDL, kMlaDR, kMlaPairs, kMlaPairSync><<<grid, kMlaPairs * 2 * kWave, 0, st>>>(a);
-    }
+    if (q_dtype == EMBER_F16)
+      launch_mfma<_Float16>(a, grid, small, four, st);
+    else
+      launch_mfma<__bf16>(a, grid, small, four, st);
     if (a.merge_apart) {
       const int64_t threads = num_seqs * num_heads * (kMlaDL / 4);
       const uint32_t blocks = static_cast<uint32_t>((threads + kWave - 1) / kWave);

@@ -101,6 +101,33 @@ def test_full_grid_two_stream_workgroups(dtype):
     assert _lib.read_errors() == 0
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("batch,heads,splits", [(150, 16, 2), (60, 16, 4), (90, 20, 3), (53, 16, 9)])
+def test_ragged_full_grids_with_stale_rows(dtype, batch, heads, splits):
+    """The register kernel's row loads and split plan at their edges: two and four tile streams,
+    one and two head chunks, contexts around a half tile, a tile and the least split (128
+    keys), an empty one, (sequence, split) counts that are no multiple of 8; a cache with
+    padded rows; every slot past a context holds NaN, which may reach no result. Three calls
+    on one workspace."""
+    g = torch.Generator().manual_seed(batch)
+    ctx_lens = torch.randint(1, 500, (batch,), generator=g).tolist()
+    ctx_lens[:14] = [1, 15, 16, 17, 32, 33, 127, 128, 129, 256, 257, 0, 1090, 2]
+    q, lat, bt, ctx = gen.mla_decode_inputs(ctx_lens, heads, DL, DR, 16, dtype, seed=batch + 1)
+    live = torch.zeros(lat.shape[:2], dtype=torch.bool)
+    for b, n in enumerate(ctx_lens):
+        for j in range(n):
+            live[bt[b, j // 16], j % 16] = True
+    cache = torch.full((lat.shape[0], 16, DL + DR + 8), float("nan"), dtype=dtype, device=DEV)[..., :DL + DR]
+    cache[live.to(DEV)] = lat[live].to(DEV)
+    rows = [b for b in range(batch) if ctx_lens[b]]
+    for _ in range(3):
+        got = mla_decode(q.to(DEV), cache, bt.to(DEV), ctx.to(DEV), SCALE, DL, num_splits=splits)
+        _check(got[rows], q[rows][..., :DL], q[rows][..., DL:], lat, bt[rows], ctx[rows], SCALE, DL, True,
+               f"B={batch} splits {splits}")
+        assert bool(torch.isnan(got[11]).all())
+    assert _lib.read_errors() == 0
+
+
 def test_long_contexts_cross_block_id_windows():
     """Contexts of 9000 and 5000 keys at one and two splits: each wave walks 40-71 tiles,
     crossing the 32-tile windows of prefetched block ids; block size 32 (two halves per
