@@ -37,6 +37,9 @@
 // silu_and_mul): Qwen3-8B 256 tokens 70.0 / 72.6, 8192 tokens 1286 / 1235; Qwen2.5-7B 256
 // tokens 110 / 88.5, 8192 tokens 1791 / 1834. The library therefore keeps the unfused pair
 // by default at these sizes and runs this kernel when the fused form is asked for.
+#include <algorithm>
+#include <type_traits>
+
 #include "ember_common.h"
 
 #ifndef EMBER_GEMM_GROUP_M
@@ -120,48 +123,15 @@ struct GemmArgs {
   int num_valid, top_k, E, ntok;
   int64_t wes;
   uint32_t* err;  // MOE: EMBER_ERR_ROW_INDEX for a valid assignment whose token is >= ntok
-  // packed weights (PK kernels only): w is the decode kernels' packed array for a grid of
+  // packed dense weights (the frag kernel): w is the decode kernels' packed array for a grid of
   // pk_G workgroups over pk_total units (pk_total = (I / 64) (H / 64))
   int64_t pk_total, pk_G;
-};
-
-// Walks the packed units of one 64-row slab, u = slab * nk + j for j = 0, 1, ...: the unit's
-// place in the packed array, tracking its owner workgroup b and b's run [start, next)
-// incrementally (a division only where the walk crosses into the next run).
-struct PackedSlabWalk {
-  int64_t u, last, b, start, next, q, total, G;
-  __device__ void init(int64_t slab, int64_t nk, int64_t total_, int64_t G_) {
-    total = total_;
-    G = G_;
-    q = total / G;
-    u = slab * nk;
-    last = u + nk - 1;
-    b = gu_owner(u, total, G);
-    start = gu_start(b, total, G);
-    next = gu_start(b + 1, total, G);
-  }
-  // the unit's element offset (16 KiB units)
-  template <typename T>
-  __device__ int64_t elem_offset() const {
-    const int64_t t = u - start;
-    const int64_t pos = t < q ? t * G + b : q * G + (start - b * q);
-    return pos * (16384 / static_cast<int64_t>(sizeof(T)));
-  }
-  __device__ void advance() {  // past the slab's last unit it stays there
-    if (u == last) return;
-    ++u;
-    if (u >= next) {
-      ++b;
-      start = next;
-      next = gu_start(b + 1, total, G);
-    }
-  }
 };
 
 template <typename T, int BNG, int BM, bool MOE, bool PK = false>
 __global__ void __launch_bounds__(512, 1)
 k_gate_up_silu_gemm(GemmArgs a) {
-  static_assert(!PK || BNG % 64 == 0, "packed tiles are whole 64-row slabs");
+  static_assert(!PK || (MOE && BNG % 64 == 0), "packed experts: tiles of whole 64-row slabs");
   using M = GemmMfma<T>;
   using V8 = typename M::v8;
   static_assert((BM == 256 && (BNG == 64 || BNG == 96 || BNG == 128)) || (BM == 128 && BNG == 128), "tile");
@@ -286,27 +256,14 @@ k_gate_up_silu_gemm(GemmArgs a) {
     }
   }
   const int nd = a.H / 64;  // double stages
-  // Dense packed weights: a unit's place depends on the decode grid it was packed for, so
-  // each slab's units are walked in k order. Routed experts' packed weights are per expert
-  // k-major (unit j * slabs + slab of the expert's array), so a stage's S units are adjacent.
-  PackedSlabWalk walk[S];
-  if (PK && !MOE) {
-#pragma unroll
-    for (int ss = 0; ss < S; ++ss) walk[ss].init(n0 / 64 + ss, nd, a.pk_total, a.pk_G);
-  }
-  // element offsets of double stage d's weight units (PK)
+  // Routed experts' packed weights are per expert k-major (unit j * slabs + slab of the
+  // expert's array), so a stage's S units are adjacent: element offsets of double stage d's.
   int64_t wofs[S];
   auto next_units = [&](int d) {
     constexpr int64_t kUnitElems = 16384 / static_cast<int64_t>(sizeof(T));
 #pragma unroll
-    for (int ss = 0; ss < S; ++ss) {
-      if (MOE) {
-        wofs[ss] = (static_cast<int64_t>(min(d, nd - 1)) * (a.I / 64) + n0 / 64 + ss) * kUnitElems;
-      } else {
-        wofs[ss] = walk[ss].template elem_offset<T>();
-        walk[ss].advance();
-      }
-    }
+    for (int ss = 0; ss < S; ++ss)
+      wofs[ss] = (static_cast<int64_t>(min(d, nd - 1)) * (a.I / 64) + n0 / 64 + ss) * kUnitElems;
   };
   auto wk = [&](int i, int kk) -> int64_t { return PK ? wofs[wsl[i]] : kk; };
   auto wbuf = [&](int d) { return lds + (SPLIT ? (d % 3) * WREG : (d % NBUF) * DST); };
@@ -444,6 +401,363 @@ k_gate_up_silu_gemm(GemmArgs a) {
   }
 }
 
+// ---------------------------------------------------------------- packed weight, dense
+//
+// k_gate_up_silu_gemm_frag: the dense GEMM over the decode kernels' packed weight. Every 1 KiB
+// block of the packed layout is one MFMA operand fragment, so the weights go from memory
+// straight to registers, one contiguous KiB per load, and only x passes through LDS. With
+// both operands in LDS (k_gate_up_silu_gemm) a 256 x (128 + 128) tile reads 192 KB and writes
+// 64 KB of LDS per 64 k, the whole of its 128 B/clk beside 2048 cycles of MFMA; here it reads
+// 128 and writes 32.
+//   * 2 CG waves in two token groups x CG column groups; a wave has BM / 2 tokens x (CW gate +
+//     CW up) columns. Waves 2c and 2c + 1 take the two token groups of one column group: they
+//     sit on different SIMDs and read the same fragments at about the same time (the second
+//     from L1).
+//   * weight fragments: a register ring of four 32-k steps, loaded three steps ahead;
+//   * x: an LDS ring of four 64-k stages, loaded two stages ahead by buffer loads to LDS (rows
+//     of 128 bytes, 16-byte chunks XOR-swizzled by row & 7). The buffer form matters: after a
+//     global_load_lds the compiler treats every wait as one for a flat access and drains both
+//     counters (vmcnt(0) lgkmcnt(0)), after a buffer load it counts;
+//   * x fragments: a register ring of four (six in 192-token tiles), each refilled behind the MFMAs that used it last;
+//   * one barrier per stage, in its middle, where the next step's operands are already in
+//     registers: no read waits for it.
+// The k order of every accumulator and the epilogue are k_gate_up_silu_gemm's, so the results
+// are its bits.
+//
+// What bounds it: the vector memory path (96 KB per 64 k of the 256 x 128 tile) beside the
+// MFMAs. Qwen3-8B, T = 8192, one box: 1353 us; without the weight loads 1171, without the x
+// loads 1244, without either 1069, MFMAs and barriers alone 1011. Deeper rings (8 and 16 weight
+// steps, 5 to 8 x stages) changed nothing, x staged through registers lost 4-10%.
+// Measured against both operands in LDS (us, bf16, the best tile of each | hipBLASLt +
+// silu_and_mul): Qwen3-8B 64 tokens 68 -> 41 | 45, 128: 69 -> 46 | 50, 200: 70 -> 60 | 63, 512:
+// 115 -> 90 | 92, 8192: 1450 -> 1320 | 1205; Qwen2.5-7B 64: 78 -> 52 | 62, 256: 100 -> 76 | 80,
+// 600: 217 -> 174 | 171; Qwen2.5-0.5B 130: 21 -> 12.3 | 12.6, 2000: 62 -> 45 | 70.
+__device__ __forceinline__ auto gemm_rsrc(const void* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, -1, kBufferWord3);
+#else
+  return p;
+#endif
+}
+// 16 bytes per lane from base + voff (per lane) + soff (uniform) to lds_base + 16 lane.
+template <typename R>
+__device__ __forceinline__ void gemm_buffer_lds16(R r, int voff, int soff, void* lds_base) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(
+                                                  reinterpret_cast<uintptr_t>(lds_base)), 16, voff, soff, 0, 0);
+#else
+  (void)r;
+  (void)voff;
+  (void)soff;
+  (void)lds_base;
+#endif
+}
+
+// Walks the packed units of one 64-row slab in k order: unit t of workgroup b's run while the
+// slab's units last. start(b) = b total / G = b q + off with q = total / G, r = total % G,
+// off = b r / G: stepping b adds r to the remainder b r % G, so the walk needs no division.
+struct SlabWalk {
+  int t, b, off, rem, len, left, q, r, G;
+  __device__ void init(int slab, int nk, int64_t total, int64_t G_) {
+    const int64_t u = static_cast<int64_t>(slab) * nk;
+    const int64_t b_ = gu_owner(u, total, G_);
+    const int64_t q_ = total / G_;
+    const int64_t start = gu_start(b_, total, G_);
+    G = __builtin_amdgcn_readfirstlane(static_cast<int>(G_));
+    q = __builtin_amdgcn_readfirstlane(static_cast<int>(q_));
+    r = __builtin_amdgcn_readfirstlane(static_cast<int>(total % G_));
+    b = __builtin_amdgcn_readfirstlane(static_cast<int>(b_));
+    t = __builtin_amdgcn_readfirstlane(static_cast<int>(u - start));
+    off = __builtin_amdgcn_readfirstlane(static_cast<int>(start - b_ * q_));
+    rem = __builtin_amdgcn_readfirstlane(static_cast<int>(b_ * (total % G_) % G_));
+    len = q + (rem + r >= G ? 1 : 0);
+    left = nk - 1;
+  }
+  __device__ int pos() const { return t < q ? t * G + b : q * G + off; }
+  // Past the slab's last unit it stays there. No branches: they would cut the k loop's body
+  // into blocks (and cost registers).
+  __device__ void advance() {
+    const int step = left > 0 ? 1 : 0;
+    left -= step;
+    t += step;
+    const int wrap = t == len ? 1 : 0;
+    t = wrap ? 0 : t;
+    b += wrap;
+    rem += wrap ? r : 0;
+    const int carry = rem >= G ? 1 : 0;
+    rem -= carry ? G : 0;
+    off += carry;
+    len = q + (rem + r >= G ? 1 : 0);
+  }
+};
+
+template <int V>
+using IntC = std::integral_constant<int, V>;
+
+template <typename T, int BM, int CG, int CW>
+__global__ void __launch_bounds__(128 * CG, (2 * CG + 3) / 4)
+k_gate_up_silu_gemm_frag(GemmArgs a) {
+  using M = GemmMfma<T>;
+  using V8 = typename M::v8;
+  constexpr int BNG = CG * CW;           // gate (and up) columns of the tile
+  constexpr int NW = 2 * CG;             // waves
+  constexpr int TW = BM / 2;             // tokens per wave
+  constexpr int NX = TW / 16;            // x fragments per 32 k
+  constexpr int NC = CW / 16;            // 16-column tiles per wave
+  constexpr int NF = 2 * NC;             // weight fragments per 32 k
+  static_assert(BM % 64 == 0 && (CW == 16 || CW == 32) && 64 % CW == 0, "a wave's columns lie in one slab");
+  constexpr int XREG = BM * kGemmRowB;   // one x stage (64 k)
+  constexpr int NBUF = 4;                // x ring: two stages of loads in flight
+  constexpr int XI = BM / 8;             // x load instructions (8 rows) per stage
+  constexpr int XL = (XI + NW - 1) / NW; // ... per wave (the last ones may repeat a row group)
+  constexpr int WR = 4;                  // weight fragment ring, in 32-k steps
+  constexpr int FX = NX % 4 == 0 ? 4 : NX;  // x fragment ring
+  static_assert(NX % FX == 0, "x fragment ring");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[NBUF * XREG];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q = w & 1;
+  const int cg = w >> 1;
+  const int n = lane & 15, g = lane >> 4;
+
+  // XCD-aware tile order, then GROUP_M token tiles per band of column tiles
+  const int mtiles = (a.T + BM - 1) / BM;
+  const int ntiles = (a.I + BNG - 1) / BNG;
+  int pid = blockIdx.x;
+  {
+    const int nb = gridDim.x;
+    const int per = (nb + 7) / 8;
+    const int xcd = pid % 8, idx = pid / 8;
+    const int full = nb % 8 == 0 ? 8 : nb % 8;
+    pid = xcd < full ? xcd * per + idx : full * per + (xcd - full) * (per - 1) + idx;
+  }
+  constexpr int GM = EMBER_GEMM_GROUP_M;
+  const int group = pid / (GM * ntiles);
+  const int first_m = group * GM;
+  const int gsize = min(mtiles - first_m, GM);
+  const int mt = first_m + (pid % (GM * ntiles)) % gsize;
+  const int nt = (pid % (GM * ntiles)) / gsize;
+  const int m0 = mt * BM, n0 = nt * BNG;
+
+  // x: byte offsets of this lane's 16 bytes from the tile's first row (padded tokens: the last
+  // real row); instruction ins moves rows 8 ins .. 8 ins + 7
+  const T* X = static_cast<const T*>(a.x) + static_cast<int64_t>(m0) * a.xs;
+  const auto xrsrc = gemm_rsrc(X);
+  const int nd = a.H / 64;
+  int src[XL], dst[XL];
+#pragma unroll
+  for (int i = 0; i < XL; ++i) {
+    const int ins = min(XL * w + i, XI - 1);
+    const int xr = 8 * ins + (lane >> 3);
+    const int c = (lane & 7) ^ (xr & 7);
+    src[i] = static_cast<int>((min(xr, a.T - 1 - m0) * a.xs + 8 * c) * static_cast<int64_t>(sizeof(T)));
+    dst[i] = ins * 1024;
+  }
+  auto issue_x = [&](int d) __attribute__((always_inline)) {
+    const int kk = min(d, nd - 1) * 64 * static_cast<int>(sizeof(T));
+#pragma unroll
+    for (int i = 0; i < XL; ++i) gemm_buffer_lds16(xrsrc, src[i], kk, lds + (d % NBUF) * XREG + dst[i]);
+  };
+  // weights: the wave's first column, the last real ones past I (nothing of those is stored)
+  const int c0 = n0 + CW * cg;
+  const int cw = min(c0, a.I - CW);
+  const unsigned char* W = static_cast<const unsigned char*>(a.w) + ((cw % 64) / 16) * 2048;
+  const uint32_t lane16 = 16u * lane;
+  SlabWalk walk;
+  walk.init(cw / 64, nd, a.pk_total, a.pk_G);
+  int64_t unit = 0;  // byte offset of the current unit
+  auto next_unit = [&]() __attribute__((always_inline)) {
+    unit = static_cast<int64_t>(walk.pos()) * 16384;
+    walk.advance();
+  };
+  V8 fw[WR][NF];
+  auto load_w = [&](V8 (&f)[NF], int half) __attribute__((always_inline)) {
+    const unsigned char* p = W + unit + half * 8192;
+#pragma unroll
+    for (int t = 0; t < NF; ++t) f[t] = *reinterpret_cast<const V8*>(p + t * 1024 + lane16);
+  };
+  const int sw = n & 7;
+  const int xrow0 = (TW * q + n) * kGemmRowB;
+  const int xo[2] = {xrow0 + ((g ^ sw) << 4), xrow0 + (((4 + g) ^ sw) << 4)};
+  V8 fx[FX];
+  auto read_x = [&](int d, int half, int u) __attribute__((always_inline)) {
+    fx[u % FX] = *reinterpret_cast<const V8*>(lds + (d % NBUF) * XREG + xo[half] + u * 16 * kGemmRowB);
+  };
+  f32x4 acc[NF][NX];
+#pragma unroll
+  for (int t = 0; t < NF; ++t)
+#pragma unroll
+    for (int u = 0; u < NX; ++u) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+  for (int i = 0; i < WR - 1; ++i) {  // weight steps 0 .. WR - 2
+    if (i % 2 == 0) next_unit();
+    load_w(fw[i], i % 2);
+  }
+#pragma unroll
+  for (int d = 0; d < NBUF - 1; ++d) issue_x(d);
+  gemm_wait_vm0();
+  gemm_barrier();
+#pragma unroll
+  for (int u = 0; u < FX; ++u) read_x(0, 0, u);
+
+  // Step 2j + H of stage j: load weight step 2j + H + WR - 1, then the MFMAs, each x fragment
+  // refilled FX groups ahead (from the next half or the next stage at the end).
+  auto step = [&](int j, auto ring, auto half) __attribute__((always_inline)) {
+    constexpr int R = decltype(ring)::value, H = decltype(half)::value;
+    constexpr int A = H + WR - 1;
+    if (A % 2 == 0) next_unit();
+    load_w(fw[(R + WR - 1) % WR], A % 2);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < NX; ++u) {
+#pragma unroll
+      for (int t = 0; t < NF; ++t) acc[t][u] = M::run(fw[R][t], fx[u % FX], acc[t][u]);
+      if (u + FX < NX) read_x(j, H, u + FX);
+      else read_x(j + H, 1 - H, u + FX - NX);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // The barrier makes x(j + 1) visible (read from step 2j + 1 on) and frees the buffer of
+  // x(j - 1) (last used by the MFMAs of step 2j - 1) for x(j + NBUF - 1). x(j + 1) was loaded
+  // before the loop or at the barrier of stage j - NBUF + 2: kYounger loads are younger.
+  constexpr int kYounger = 2 * (NBUF - 2) * NF + (NBUF - 3) * XL;
+  static_assert(kYounger < 64, "vmcnt");
+  auto stage = [&](int j, auto ring) __attribute__((always_inline)) {
+    constexpr int R = decltype(ring)::value;
+    step(j, IntC<R>{}, IntC<0>{});
+    gemm_wait_vm<kYounger>();
+    gemm_barrier();
+    issue_x(j + NBUF - 1);
+    step(j, IntC<(R + 1) % WR>{}, IntC<1>{});
+  };
+  int j = 0;
+  for (; j + 2 <= nd; j += 2) {
+    stage(j, IntC<0>{});
+    stage(j + 1, IntC<2>{});
+  }
+  if (j < nd) stage(j, IntC<0>{});
+  gemm_wait_vm0();
+
+  // Epilogue: lane (n, g) holds rows 4g + r of each 16-row tile for token 16 u + n.
+  if (c0 >= a.I) return;
+  T* out = static_cast<T*>(a.out);
+#pragma unroll
+  for (int u = 0; u < NX; ++u) {
+    const int tok = m0 + TW * q + 16 * u + n;
+    if (tok < a.T) {
+#pragma unroll
+      for (int t = 0; t < NC; ++t) {
+        Pack<T, 4> o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float gf = round_to<T>(acc[2 * t][u][r]);
+          const float uf = round_to<T>(acc[2 * t + 1][u][r]);
+          const float act = round_to<T>(gf / (1.0f + expf(-gf)));
+          o.v[r] = half_product<T>(act, uf);
+        }
+        store_pack<T, 4>(out + static_cast<int64_t>(tok) * a.os + c0 + 16 * t + 4 * g, o);
+      }
+    }
+  }
+}
+
+template <typename T, int BM, int CG, int CW>
+int launch_frag(const GemmArgs& a, hipStream_t st) {
+  const int64_t grid = cdiv(a.T, BM) * cdiv(a.I, CG * CW);
+  if (grid > 0x7fffffffLL) return EMBER_EINVAL;
+  k_gate_up_silu_gemm_frag<T, BM, CG, CW><<<dim3(static_cast<uint32_t>(grid)), dim3(128 * CG), 0, st>>>(a);
+  return launch_status();
+}
+
+// A tile's workgroup takes about as long as the rows it streams, BM x rows and 2 x columns
+// weight rows per k, whatever their split (us per round of tiles at H = 4096; rows: 224 41-46,
+// 256 45-50, 288 53-56, 320 60-63, 352 55-61, 384 56-72, 448 70-88, 512 87-111): the tile with
+// the fewest rows in all rounds, the smaller on a tie. The
+// 192-token tiles: Qwen3-8B 160 tokens 60 -> 51 us, 300: 89 -> 70, 700: 164 -> 134.
+void frag_pick_tile(int64_t tokens, int64_t inter, int64_t& token_tile, int64_t& column_tile) {
+  const int64_t ncu = std::max(1, device_cu_count());
+  int64_t best = INT64_MAX;
+  for (int64_t bm : {128, 192, 256})
+    for (int64_t cols : {32, 48, 64, 80, 96, 128}) {
+      if (bm > 128 && cols == 32) continue;  // four waves of 96 or 128 tokens: slower than their rows
+      const int64_t rows = cdiv(cdiv(tokens, bm) * cdiv(inter, cols), ncu) * (bm + 2 * cols);
+      if (rows < best) {
+        best = rows;
+        token_tile = bm;
+        column_tile = cols;
+      }
+    }
+}
+
+template <typename T>
+int launch_frag_tile(const GemmArgs& a, int64_t token_tile, int64_t column_tile, hipStream_t st) {
+  if (token_tile == 128) {
+    switch (column_tile) {
+      case 32: return launch_frag<T, 128, 2, 16>(a, st);
+      case 48: return launch_frag<T, 128, 3, 16>(a, st);
+      case 64: return launch_frag<T, 128, 4, 16>(a, st);
+      case 80: return launch_frag<T, 128, 5, 16>(a, st);
+      case 96: return launch_frag<T, 128, 6, 16>(a, st);
+      default: return launch_frag<T, 128, 4, 32>(a, st);
+    }
+  }
+  if (token_tile == 192) {
+    switch (column_tile) {
+      case 48: return launch_frag<T, 192, 3, 16>(a, st);
+      case 64: return launch_frag<T, 192, 4, 16>(a, st);
+      case 80: return launch_frag<T, 192, 5, 16>(a, st);
+      case 96: return launch_frag<T, 192, 6, 16>(a, st);
+      default: return launch_frag<T, 192, 4, 32>(a, st);
+    }
+  }
+  switch (column_tile) {
+    case 48: return launch_frag<T, 256, 3, 16>(a, st);
+    case 64: return launch_frag<T, 256, 4, 16>(a, st);
+    case 80: return launch_frag<T, 256, 5, 16>(a, st);
+    case 96: return launch_frag<T, 256, 6, 16>(a, st);
+    default: return launch_frag<T, 256, 4, 32>(a, st);
+  }
+}
+
+// The packed entry points' body: token_tile 0 lets frag_pick_tile choose.
+int gemm_packed_core(const void* x, int64_t x_row_stride, const void* packed, int dtype, int64_t tokens,
+                     int64_t hidden, int64_t inter, int64_t num_workgroups, int64_t token_tile, int64_t column_tile,
+                     void* out, int64_t out_row_stride, void* stream) {
+  if (tokens == 0) return EMBER_OK;
+  if (tokens < 0 || tokens > (int64_t(1) << 24) || hidden < 64 || hidden % 64 != 0 || hidden > (int64_t(1) << 20) ||
+      inter < 64 || inter % 64 != 0 || inter > (int64_t(1) << 28) || num_workgroups < 1)
+    return EMBER_EINVAL;
+  const bool shape = (token_tile == 256 && (column_tile == 64 || column_tile == 128)) ||
+                     (token_tile == 128 && column_tile == 128);
+  if (token_tile != 0 && (!shape || inter % column_tile != 0)) return EMBER_EINVAL;
+  if (dtype != EMBER_F16 && dtype != EMBER_BF16) return EMBER_EINVAL;
+  if (x == nullptr || packed == nullptr || out == nullptr || !aligned16(x) || !aligned16(packed) || !aligned16(out))
+    return EMBER_EINVAL;
+  if (x_row_stride < hidden || out_row_stride < inter || x_row_stride % 8 != 0 || out_row_stride % 4 != 0)
+    return EMBER_EINVAL;
+  const int64_t total = (inter / 64) * (hidden / 64);
+  if (total > INT32_MAX) return EMBER_EINVAL;  // 32 TiB of weights
+  // A tile's rows are addressed by 32-bit offsets: rows farther apart than that allows go in
+  // calls of one token.
+  constexpr int64_t kMaxStride = int64_t(1) << 22;
+  const int64_t per_call = x_row_stride > kMaxStride ? 1 : tokens;
+  if (token_tile == 0) frag_pick_tile(per_call, inter, token_tile, column_tile);
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  for (int64_t t = 0; t < tokens; t += per_call) {
+    const GemmArgs a{static_cast<const char*>(x) + 2 * t * x_row_stride, x_row_stride, packed, 0,
+                     static_cast<char*>(out) + 2 * t * out_row_stride, out_row_stride, static_cast<int>(per_call),
+                     static_cast<int>(hidden), static_cast<int>(inter), nullptr, nullptr, 0, 1, 0, 0, 0, nullptr,
+                     total, num_workgroups < total ? num_workgroups : total};  // the packing's grid
+    const int rc = dtype == EMBER_F16 ? launch_frag_tile<_Float16>(a, token_tile, column_tile, st)
+                                      : launch_frag_tile<__bf16>(a, token_tile, column_tile, st);
+    if (rc != EMBER_OK) return rc;
+  }
+  return EMBER_OK;
+}
+
 template <typename T, int BNG, int BM = 256, bool MOE = false, bool PK = false>
 int launch_gemm(const GemmArgs& a, hipStream_t st) {
   const int64_t grid = cdiv(a.T, BM) * cdiv(a.I, BNG);
@@ -528,32 +842,16 @@ extern "C" int ember_gate_up_silu_gemm_packed(const void* x, int64_t x_row_strid
                                               int64_t tokens, int64_t hidden, int64_t inter, int64_t num_workgroups,
                                               int64_t token_tile, int64_t column_tile, void* out,
                                               int64_t out_row_stride, void* stream) {
-  using namespace ember;
-  if (tokens == 0) return EMBER_OK;
-  if (tokens < 0 || tokens > (int64_t(1) << 24) || hidden < 64 || hidden % 64 != 0 || hidden > (int64_t(1) << 20) ||
-      inter < 64 || inter % 64 != 0 || inter > (int64_t(1) << 28) || num_workgroups < 1)
-    return EMBER_EINVAL;
-  const bool shape = (token_tile == 256 && (column_tile == 64 || column_tile == 128)) ||
-                     (token_tile == 128 && column_tile == 128);
-  if (!shape || inter % column_tile != 0) return EMBER_EINVAL;
-  if (dtype != EMBER_F16 && dtype != EMBER_BF16) return EMBER_EINVAL;
-  if (x == nullptr || packed == nullptr || out == nullptr || !aligned16(x) || !aligned16(packed) || !aligned16(out))
-    return EMBER_EINVAL;
-  if (x_row_stride < hidden || out_row_stride < inter || x_row_stride % 8 != 0 || out_row_stride % 4 != 0)
-    return EMBER_EINVAL;
-  const int64_t total = (inter / 64) * (hidden / 64);
-  GemmArgs a{x, x_row_stride, packed, 0, out, out_row_stride, static_cast<int>(tokens),
-             static_cast<int>(hidden), static_cast<int>(inter), nullptr, nullptr, 0, 1, 0, 0, 0, nullptr,
-             total, num_workgroups < total ? num_workgroups : total};  // the packing's grid
-  const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (dtype == EMBER_F16) {
-    if (token_tile == 128) return launch_gemm<_Float16, 128, 128, false, true>(a, st);
-    return column_tile == 64 ? launch_gemm<_Float16, 64, 256, false, true>(a, st)
-                             : launch_gemm<_Float16, 128, 256, false, true>(a, st);
-  }
-  if (token_tile == 128) return launch_gemm<__bf16, 128, 128, false, true>(a, st);
-  return column_tile == 64 ? launch_gemm<__bf16, 64, 256, false, true>(a, st)
-                           : launch_gemm<__bf16, 128, 256, false, true>(a, st);
+  return ember::gemm_packed_core(x, x_row_stride, packed, dtype, tokens, hidden, inter, num_workgroups,
+                                 token_tile > 0 ? token_tile : -1, column_tile, out, out_row_stride, stream);
+}
+
+extern "C" int ember_gate_up_silu_gemm_packed_auto(const void* x, int64_t x_row_stride, const void* packed, int dtype,
+                                                   int64_t tokens, int64_t hidden, int64_t inter,
+                                                   int64_t num_workgroups, void* out, int64_t out_row_stride,
+                                                   void* stream) {
+  return ember::gemm_packed_core(x, x_row_stride, packed, dtype, tokens, hidden, inter, num_workgroups, 0, 0, out,
+                                 out_row_stride, stream);
 }
 
 extern "C" int ember_moe_gate_up_silu_gemm_packed(const void* x, int64_t x_row_stride, int64_t num_tokens,

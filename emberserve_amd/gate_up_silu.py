@@ -19,8 +19,9 @@ prefill-size MFMA GEMM with the activation as its epilogue, `gate_up_silu_gemm`,
 never materialises the [T, 2I] projection) and `fused=False` the pair. Over a weight packed at load time (`packed=`) the kernel runs by
 default up to PACKED_FUSED_TOKENS: 35.3 vs 46.1 us at 16 tokens and 37.1 vs 45.8 at 32
 (Qwen3-8B), 52.0 vs 56.7 at 32 (Qwen2.5-7B); at 48-64 tokens it is ahead at Qwen3-8B
-(44.5 vs 47.8) and behind at Qwen2.5-7B (65.0 vs 63.0). Where the kernel does not apply (more than 64 tokens, fp32, shapes
-that are not multiples of 64, unaligned operands) the pair runs. CPU tensors, or
+(44.5 vs 47.8) and behind at Qwen2.5-7B (65.0 vs 63.0). Above that the packed GEMM runs by
+default where `packed_gemm_default` says so, else the pair. Where no kernel applies (fp32,
+shapes that are not multiples of 64, unaligned operands) the pair runs. CPU tensors, or
 `EMBERSERVE_FUSED_OPS=0`, take the eager forms.
 
 The kernel is persistent: `num_workgroups` workgroups (default one per CU) take equal runs
@@ -191,14 +192,22 @@ def gate_up_silu_gemm(x: Tensor, weight: Tensor, *, column_tile: int = 128, toke
     return out.view(*x.shape[:-1], I)
 
 
-PACKED_GEMM_TILES = (64, 128)  # the packed GEMM's column tiles: whole 64-row slabs
+def _launch_gemm_packed(x2: Tensor, packed: PackedGateUp, out: Tensor) -> None:
+    _launch("ember_gate_up_silu_gemm_packed_auto", _lib.load().ember_gate_up_silu_gemm_packed_auto, x2.device,
+            x2.data_ptr(), x2.stride(0), packed.packed.data_ptr(), _lib.dtype_tag(x2.dtype), x2.shape[0],
+            packed.hidden, packed.inter, packed.num_workgroups, out.data_ptr(), out.stride(0))
+
+
+PACKED_GEMM_TILES = (64, 128)  # the column tiles gate_up_silu_gemm_packed can be asked for
 
 
 def gate_up_silu_gemm_packed(x: Tensor, packed: PackedGateUp, *, column_tile: int | None = None,
                              token_tile: int = 256) -> Tensor:
     """gate_up_silu_gemm over the packed weight (`ember_gate_up_silu_gemm_packed`): the same
-    tiles but the 96-column one, the same results bit for bit. With it the packed copy is
-    the only gate_up weight a model needs (decode kernels and prefill read it)."""
+    results bit for bit at every tile. column_tile None (with the default token_tile) leaves
+    the tile to the library (`ember_gate_up_silu_gemm_packed_auto`); otherwise the tiles of
+    gate_up_silu_gemm but the 96-column one. With it the packed copy is the only gate_up
+    weight a model needs (decode kernels and prefill read it)."""
     H, I = packed.hidden, packed.inter
     if x.shape[-1] != H or x.dtype != packed.dtype:
         raise ValueError(f"gate_up_silu_gemm_packed: x {tuple(x.shape)} {x.dtype} does not match the packed "
@@ -209,16 +218,31 @@ def gate_up_silu_gemm_packed(x: Tensor, packed: PackedGateUp, *, column_tile: in
     out = torch.empty((T, I), dtype=x.dtype, device=x.device)
     if T == 0:
         return out.view(*x.shape[:-1], I)
+    auto = column_tile is None and token_tile == 256
     if column_tile is None:
-        column_tile = gemm_column_tile(T, I, x.device, PACKED_GEMM_TILES)
+        column_tile = 64 if auto else gemm_column_tile(T, I, x.device, PACKED_GEMM_TILES)
     if not (T <= 1 << 24 and x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and x2.data_ptr() % 16 == 0
             and (token_tile, column_tile) in ((256, 64), (256, 128), (128, 128)) and I % column_tile == 0):
         raise ValueError(f"gate_up_silu_gemm_packed: shape, stride or tile not supported (I {I}, "
                          f"column_tile {column_tile}, token_tile {token_tile})")
+    if auto:
+        _launch_gemm_packed(x2, packed, out)
+        return out.view(*x.shape[:-1], I)
     _launch("ember_gate_up_silu_gemm_packed", _lib.load().ember_gate_up_silu_gemm_packed, x.device,
             x2.data_ptr(), x2.stride(0), packed.packed.data_ptr(), _lib.dtype_tag(x.dtype), T, H, I,
             packed.num_workgroups, token_tile, column_tile, out.data_ptr(), out.stride(0))
     return out.view(*x.shape[:-1], I)
+
+
+def packed_gemm_default(tokens: int, hidden: int, inter: int, device: torch.device) -> bool:
+    """Whether the packed GEMM runs by default above PACKED_FUSED_TOKENS when the unpacked
+    weight is there too: while its tiles fit the CUs in one round, and at any size for short
+    rows, where the projection's round trip through memory is long against its product.
+    Measured (bf16, us, packed GEMM | hipBLASLt + silu_and_mul): Qwen3-8B 64 tokens 41 | 45,
+    128: 46 | 50, 160: 51 | 55, 200: 60 | 63, 256: 63 | 65, 300: 70 | 76, 512: 90 | 91, but 2048: 317 | 301;
+    Qwen2.5-7B 64: 51 | 62, 128: 56 | 70, 256: 80 | 82, but 600: 188 | 172; Qwen2.5-0.5B (H 896)
+    100: 9.3 | 13, 1024: 27 | 37, 8192: 161 | 199."""
+    return hidden <= 1024 or -(-tokens // 256) * -(-inter // 128) <= num_sms(device)
 
 
 def gate_up_silu(x: Tensor, weight: Tensor | None, *, num_workgroups: int | None = None,
@@ -226,14 +250,15 @@ def gate_up_silu(x: Tensor, weight: Tensor | None, *, num_workgroups: int | None
     """silu_and_mul(F.linear(x, weight)) with weight [2I, H] (qwen2.py:60-61). With `packed`
     (`pack_gate_up_weight(weight)`), the fused kernel reads the packed copy instead. With
     `packed` and weight None (a model that dropped the unpacked weight) every size runs on
-    the packed copy: the decode kernel up to PACKED_MAX_TOKENS tokens, the packed prefill
-    GEMM above."""
+    the packed copy: the decode kernel up to PACKED_FUSED_TOKENS tokens, the packed prefill
+    GEMM above (33-64 tokens, us, decode kernel | GEMM: Qwen3-8B 39-42 | 40-41, Qwen2.5-7B 63-68
+    | 50, Qwen2.5-0.5B 12 | 9)."""
     if weight is None:
         if packed is None:
             raise ValueError("gate_up_silu: weight None needs the packed weight")
         if fused is False:
             raise ValueError("gate_up_silu: the unfused pair needs the unpacked weight")
-        if x.reshape(-1, packed.hidden).shape[0] > PACKED_MAX_TOKENS:
+        if x.reshape(-1, packed.hidden).shape[0] > PACKED_FUSED_TOKENS:
             return gate_up_silu_gemm_packed(x, packed)
         return _packed_decode(x, packed, num_workgroups)
     return _gate_up_silu_decode(x, weight, num_workgroups, fused, packed)
@@ -293,6 +318,11 @@ def _gate_up_silu_decode(x: Tensor, weight: Tensor, num_workgroups: int | None, 
     if fused is True and T > limit and _gemm_fits(x2, weight, out) and any(_tile_ok(I, t) for t in GEMM_TILES):
         # the fused form asked for at prefill sizes: the MFMA GEMM with the activation epilogue
         return gate_up_silu_gemm(x, weight, column_tile=gemm_column_tile(T, I, x.device))
+    if (fused is None and T > default and packed is not None and num_workgroups is None
+            and _gemm_fits(x2, weight, out) and packed_gemm_default(T, H, I, x.device)
+            and (packed.hidden, packed.inter, packed.dtype, packed.device) == (H, I, x.dtype, x.device)):
+        _launch_gemm_packed(x2, packed, out)
+        return out.view(*x.shape[:-1], I)
     if fused is False or (fused is None and T > default) or not _fits(x2, weight, out, limit):
         return gate_up_silu_torch(x, weight)
     programs = gate_up_silu_workgroups(x.device) if num_workgroups is None else int(num_workgroups)

@@ -519,14 +519,21 @@ int ember_gate_up_silu_packed(const void* x, int64_t x_row_stride, const void* p
 /* ember_gate_up_silu_gemm over a weight packed by ember_gate_up_silu_pack_weight for
  * num_workgroups decode workgroups: the same tiles without the 96-column one ((256, 64),
  * (256, 128), (128, 128); inter a multiple of column_tile), the same results bit for bit.
- * Each tile's weight operand is its 64-row slabs' packed 16 KiB units, read as contiguous
- * 1 KiB blocks. With it a model keeps one copy of the gate_up weight (the packed one) for
+ * The weights go from memory to registers as the units' contiguous 1 KiB operand blocks;
+ * only x is staged in LDS. With it a model keeps one copy of the gate_up weight (the packed one) for
  * both the decode kernels and prefill. Replaces qwen2.py:60-61 (gate_up_proj, then
  * silu_and_mul); num_workgroups must be the value the weight was packed for. */
 int ember_gate_up_silu_gemm_packed(const void* x, int64_t x_row_stride, const void* packed, int dtype,
                                    int64_t tokens, int64_t hidden, int64_t inter, int64_t num_workgroups,
                                    int64_t token_tile, int64_t column_tile, void* out, int64_t out_row_stride,
                                    void* stream);
+
+/* ember_gate_up_silu_gemm_packed at the tile the library picks for the shape and this GPU
+ * (128, 192 or 256 tokens x 32 to 128 columns; any inter that is a multiple of 64): the same
+ * results bit for bit. */
+int ember_gate_up_silu_gemm_packed_auto(const void* x, int64_t x_row_stride, const void* packed, int dtype,
+                                        int64_t tokens, int64_t hidden, int64_t inter, int64_t num_workgroups,
+                                        void* out, int64_t out_row_stride, void* stream);
 
 /* ember_moe_gate_up_silu_gemm over experts packed by ember_moe_gate_up_silu_pack_weight
  * (tiles (256, 64), (256, 128), (128, 128); inter a multiple of column_tile): the same

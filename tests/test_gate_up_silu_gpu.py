@@ -305,6 +305,26 @@ def test_gemm_packed_equals_the_gemm(token_tile, tile, programs):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hidden,inter,programs", [(64, 64, 7), (192, 192, 5), (320, 1088, 64), (896, 4864, 256),
+                                                   (1024, 12288, 192)])
+def test_gemm_packed_auto_tiles(dtype, hidden, inter, programs):
+    """The packed GEMM at the tile the library picks: token counts around the tokens of a
+    fragment, a wave and both tiles, one and odd 64-k stages, column tiles that are ragged at
+    I, weights packed for grids whose runs split slabs; x with padded rows. Equal to the
+    unpacked GEMM bit for bit."""
+    from emberserve_amd.gate_up_silu import gate_up_silu_gemm, gate_up_silu_gemm_packed, pack_gate_up_weight
+    g = torch.Generator().manual_seed(hidden + inter)
+    w = (torch.randn(2 * inter, hidden, generator=g) / hidden ** 0.5).to(dtype).to(DEV)
+    packed = pack_gate_up_weight(w, programs)
+    for tokens in (1, 15, 17, 63, 64, 65, 127, 129, 200, 256, 257, 400, 1025):
+        _say(f"packed auto H={hidden} I={inter} T={tokens} {dtype}")
+        x = (torch.randn(tokens, hidden + 8, generator=g) * 0.5).to(dtype).to(DEV)[:, :hidden]
+        want = gate_up_silu_gemm(x, w, column_tile=64)
+        got = gate_up_silu_gemm_packed(x, packed)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), tokens
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_gemm_packed_qwen3_8b_against_oracle(dtype):
     """Qwen3-8B's MLP (H 4096, I 12288) at 777 tokens over a weight packed for the default
     grid: equal to the unpacked GEMM, and sampled rows and columns against the oracle."""
