@@ -31,6 +31,22 @@ _DTYPE_TAG = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
 
+
+class _NoFast:
+    """Stands in for the native host path while it is not built: every call is left to the
+    Python wrappers, which fail in load() on the first GPU call."""
+
+    ABI_VERSION = None
+
+    def __getattr__(self, name: str):
+        return lambda *args: None
+
+
+try:
+    from . import _fast as fast  # the native host path (csrc/fast_ops.cpp); unbound until load()
+except ImportError:
+    fast = _NoFast()
+
 _p = ctypes.c_void_p
 _i64 = ctypes.c_int64
 _i32 = ctypes.c_int
@@ -127,6 +143,10 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
         if got != ABI_VERSION:
             raise RuntimeError(f"emberserve_amd: {p} has ABI version {got}, expected {ABI_VERSION}; rebuild it")
         if path is None:
+            if fast.ABI_VERSION != ABI_VERSION:
+                raise RuntimeError(f"emberserve_amd: _fast.so is not built or has ABI version {fast.ABI_VERSION} "
+                                   f"(expected {ABI_VERSION}); run `python -m emberserve_amd.build`")
+            fast.bind({name: ctypes.cast(getattr(lib, name), _p).value for name in SIGNATURES})
             _lib = lib
         return lib
 

@@ -1,7 +1,9 @@
-"""Builds libember_ops.so (the gfx950 HIP kernels behind the C ABI in include/ember_ops.h).
+"""Builds libember_ops.so (the gfx950 HIP kernels behind the C ABI in include/ember_ops.h) and
+_fast.so (the ops' native host path, a CPython extension over torch's C++ API).
 
 `python -m emberserve_amd.build` or `build()` compiles every `csrc/*.hip` with hipcc for
-gfx950, in parallel, and links the shared library next to this file, where `_lib` loads it.
+gfx950, in parallel, and links the shared library next to this file, where `_lib` loads it;
+csrc/fast_ops.cpp is compiled by the host compiler beside them.
 No GPU is needed: hipcc cross-compiles.
 """
 
@@ -12,12 +14,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 BUILD_DIR = PKG_DIR / "_build"
 LIB_PATH = PKG_DIR / "libember_ops.so"
+FAST_PATH = PKG_DIR / "_fast.so"
 ARCH = "gfx950"
 
 # -ffp-contract=off: a*b+c stays two rounded operations, as in the reference's separate
@@ -47,14 +51,37 @@ def _compile(src: Path, obj: Path) -> None:
         raise RuntimeError(f"hipcc failed on {src.name}:\n{res.stderr}")
 
 
+def _build_fast() -> None:
+    """Compiles csrc/fast_ops.cpp into _fast.so."""
+    import torch
+
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        raise RuntimeError("no C++ compiler found (set CXX)")
+    rocm = Path(hipcc()).resolve().parent.parent
+    inc = Path(torch.__file__).resolve().parent / "include"
+    lib = inc.parent / "lib"
+    tmp = FAST_PATH.with_suffix(".so.tmp")
+    cmd = [*cxx.split(), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{inc}",
+           f"-I{inc / 'torch/csrc/api/include'}", f"-I{sysconfig.get_paths()['include']}", f"-I{rocm / 'include'}",
+           str(CSRC / "fast_ops.cpp"), "-o", str(tmp), f"-L{lib}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
+           "-lc10_hip"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{cxx} failed on fast_ops.cpp:\n{res.stderr}")
+    os.replace(tmp, FAST_PATH)
+
+
 def build(verbose: bool = False) -> Path:
-    """Compiles every kernel source and links `libember_ops.so`; returns its path."""
+    """Compiles every kernel source, links `libember_ops.so` and builds `_fast.so`; returns
+    the library's path."""
     BUILD_DIR.mkdir(exist_ok=True)
     sources = sorted(CSRC.glob("*.hip"))
     objs = [BUILD_DIR / (s.stem + ".o") for s in sources]
     workers = min(len(sources), int(os.environ.get("MAX_JOBS", os.cpu_count() or 4)), 16)
     with concurrent.futures.ThreadPoolExecutor(max_workers=max(1, workers)) as ex:
-        futs = [ex.submit(_compile, s, o) for s, o in zip(sources, objs)]
+        futs = [ex.submit(_build_fast)] + [ex.submit(_compile, s, o) for s, o in zip(sources, objs)]
         for f in futs:
             f.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")

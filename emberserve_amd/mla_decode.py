@@ -73,6 +73,15 @@ def _workspace_bytes(num_splits: int, batch: int, num_heads: int, dl: int) -> in
 _SCRATCH = ScratchCache("mla_decode", min_bytes=16)
 
 
+def _plan(B: int, H: int, DL: int, max_context: int, q_c: Tensor) -> tuple[int, Tensor | None]:
+    """The default split count and its workspace for the native host path."""
+    splits = mla_num_splits(B, q_c.device, num_heads=H, max_context=max_context)
+    splits = max(1, min(splits, max(1, -(-max_context // TILE))))
+    if splits == 1:
+        return 1, None
+    return splits, _SCRATCH.get((splits, B, H, DL), lambda: _workspace_bytes(splits, B, H, DL), q_c.device)
+
+
 def mla_decode_torch(q_c: Tensor, q_pe: Tensor, latent_cache: Tensor, block_tables: Tensor,
                      context_lens: Tensor, scale: float, kv_lora_rank: int) -> Tensor:
     """mla_attention_absorbed with identity W_UK / W_UV per sequence (mla_torch.py:33-53)
@@ -105,6 +114,10 @@ def mla_decode(q_abs: Tensor | tuple[Tensor, Tensor], latent_cache: Tensor, bloc
     else:
         q_c, q_pe = q_abs[..., :DL], q_abs[..., DL:]
         D = q_abs.shape[2]
+    if num_splits is None and out is None and q_c.dim() == 3 and q_c.shape[2] == DL:
+        got = _lib.fast.mla_decode(q_c, q_pe, latent_cache, block_tables, context_lens, scale, _plan)
+        if got is not None:  # an ordinary call, answered by the native host path
+            return got
     B, H = q_c.shape[:2]
     num_blocks, block_size, Dl = latent_cache.shape
     DR = D - DL

@@ -31,6 +31,7 @@ import os
 import torch
 
 from . import _lib
+from ._lib import fast
 from .eager import (  # noqa: F401  (re-exported: the reference's names)
     _rotate_half,
     embedding_torch,
@@ -498,8 +499,15 @@ def mla_latent_rope_cache_hip(c: torch.Tensor, k_pe: torch.Tensor, q_pe: torch.T
 
 
 # ---- dispatch (ops.py:92-115 plus the fused additions) ----------------------------------
+#
+# An ordinary GPU call is answered by the native host path (`fast`, csrc/fast_ops.cpp), which
+# returns None, with nothing launched, for every other one: CPU tensors, the opt-out, index
+# checks, operands that need a conversion, and whatever is to be refused.
 
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
+    got = fast.rmsnorm(x, weight, eps)
+    if got is not None:
+        return got
     if fused_enabled(x):
         return rmsnorm_hip(x, weight, eps)
     return rmsnorm_torch(x, weight, eps)
@@ -507,6 +515,9 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
 
 def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
                       eps: float) -> tuple[torch.Tensor, torch.Tensor]:
+    got = fast.add_rmsnorm(x, residual, weight, eps)
+    if got is not None:
+        return got
     if fused_enabled(x):
         return fused_add_rmsnorm_hip(x, residual, weight, eps)
     return fused_add_rmsnorm_torch(x, residual, weight, eps)
@@ -514,18 +525,27 @@ def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Ten
 
 def rope(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
          positions: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    got = fast.rope(q, k, cos, sin, positions)
+    if got is not None:
+        return got
     if fused_enabled(q):
         return rope_hip(q, k, cos, sin, positions)
     return rope_torch(q, k, cos, sin, positions)
 
 
 def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
+    got = fast.silu_and_mul(x)
+    if got is not None:
+        return got
     if fused_enabled(x):
         return silu_and_mul_hip(x)
     return silu_and_mul_torch(x)
 
 
 def embedding(ids: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    got = fast.embedding(ids, weight)
+    if got is not None:
+        return got
     if fused_enabled(weight):
         return embedding_hip(ids, weight)
     return embedding_torch(ids, weight)
@@ -534,6 +554,9 @@ def embedding(ids: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 def qk_norm_rope(q: torch.Tensor, k: torch.Tensor, q_weight: torch.Tensor, k_weight: torch.Tensor,
                  eps: float, cos: torch.Tensor, sin: torch.Tensor,
                  positions: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    got = fast.qk_norm_rope(q, k, q_weight, k_weight, eps, cos, sin, positions)
+    if got is not None:
+        return got
     if fused_enabled(q):
         return qk_norm_rope_hip(q, k, q_weight, k_weight, eps, cos, sin, positions)
     return qk_norm_rope_torch(q, k, q_weight, k_weight, eps, cos, sin, positions)
@@ -542,6 +565,9 @@ def qk_norm_rope(q: torch.Tensor, k: torch.Tensor, q_weight: torch.Tensor, k_wei
 def mla_latent_rope(c: torch.Tensor, k_pe: torch.Tensor, q_pe: torch.Tensor, weight: torch.Tensor,
                     eps: float, cos: torch.Tensor, sin: torch.Tensor,
                     positions: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    got = fast.mla_latent_rope(c, k_pe, q_pe, weight, eps, cos, sin, positions)
+    if got is not None:
+        return got
     if fused_enabled(c):
         return mla_latent_rope_hip(c, k_pe, q_pe, weight, eps, cos, sin, positions)
     return mla_latent_rope_torch(c, k_pe, q_pe, weight, eps, cos, sin, positions)
@@ -564,6 +590,10 @@ def rope_kv_cache(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.
                   positions: torch.Tensor, slot_mapping: torch.Tensor, k_cache: torch.Tensor,
                   v_cache: torch.Tensor, q_weight: torch.Tensor | None = None,
                   k_weight: torch.Tensor | None = None, eps: float = 1e-6) -> tuple[torch.Tensor, torch.Tensor]:
+    got = fast.rope_kv_cache(q, k, v, cos, sin, positions, slot_mapping, k_cache, v_cache, q_weight, k_weight,
+                             eps)
+    if got is not None:
+        return got
     if fused_enabled(q):
         return rope_kv_cache_hip(q, k, v, cos, sin, positions, slot_mapping, k_cache, v_cache, q_weight,
                                  k_weight, eps)
@@ -579,6 +609,10 @@ def mla_latent_rope_cache(c: torch.Tensor, k_pe: torch.Tensor, q_pe: torch.Tenso
                           eps: float, cos: torch.Tensor, sin: torch.Tensor, positions: torch.Tensor,
                           slot_mapping: torch.Tensor, cache: torch.Tensor,
                           return_latent: bool = True) -> tuple[torch.Tensor, torch.Tensor | None]:
+    got = fast.mla_latent_rope_cache(c, k_pe, q_pe, weight, eps, cos, sin, positions, slot_mapping, cache,
+                                     return_latent)
+    if got is not None:
+        return got
     if fused_enabled(c):
         return mla_latent_rope_cache_hip(c, k_pe, q_pe, weight, eps, cos, sin, positions, slot_mapping, cache,
                                          return_latent)

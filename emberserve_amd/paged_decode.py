@@ -131,6 +131,15 @@ def _workspace_bytes(num_splits: int, batch: int, num_heads: int, head_dim: int)
 _SCRATCH = ScratchCache("paged_attention_decode", min_bytes=16)
 
 
+def _plan(B: int, H: int, D: int, Hkv: int, max_context: int, q: Tensor) -> tuple[int, Tensor | None]:
+    """The default split count and its workspace for the native host path."""
+    splits = default_num_splits(B, Hkv, max_context, q.device, H, D)
+    splits = max(1, min(splits, max(1, -(-max_context // TILE))))
+    if splits == 1:
+        return 1, None
+    return splits, _SCRATCH.get((splits, B, H, D), lambda: _workspace_bytes(splits, B, H, D), q.device)
+
+
 def paged_decode_torch(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_tables: Tensor,
                        context_lens: Tensor, scale: float) -> Tensor:
     """PagedTorchAttentionBackend._decode (attn/paged_torch.py:87-98) over the gather of
@@ -160,6 +169,10 @@ def paged_attention_decode(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_ta
     """One-token-per-sequence paged attention (paged_triton.py:323-399). `num_warps` is
     accepted for signature compatibility; the kernel's workgroup shape is fixed."""
     del num_warps
+    if num_splits is None and out is None and variant is None:
+        got = _lib.fast.paged_decode(q, k_cache, v_cache, block_tables, context_lens, scale, _plan)
+        if got is not None:  # an ordinary call, answered by the native host path
+            return got
     B, H, D = q.shape
     num_blocks, block_size, Hkv, Dk = k_cache.shape
     assert Dk == D and v_cache.shape == k_cache.shape, (q.shape, k_cache.shape, v_cache.shape)
