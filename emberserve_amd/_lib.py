@@ -32,20 +32,16 @@ _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
 
 
-class _NoFast:
-    """Stands in for the native host path while it is not built: every call is left to the
-    Python wrappers, which fail in load() on the first GPU call."""
-
-    ABI_VERSION = None
+class _Fast:
+    """The native host path (csrc/fast_ops.cpp). load() fills it with the functions of _fast.so;
+    until then every call is left to the Python wrappers, whose first GPU call runs load(). The
+    extension is not imported before that, so a process may import the package, build, and load."""
 
     def __getattr__(self, name: str):
         return lambda *args: None
 
 
-try:
-    from . import _fast as fast  # the native host path (csrc/fast_ops.cpp); unbound until load()
-except ImportError:
-    fast = _NoFast()
+fast = _Fast()
 
 _p = ctypes.c_void_p
 _i64 = ctypes.c_int64
@@ -143,10 +139,16 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
         if got != ABI_VERSION:
             raise RuntimeError(f"emberserve_amd: {p} has ABI version {got}, expected {ABI_VERSION}; rebuild it")
         if path is None:
-            if fast.ABI_VERSION != ABI_VERSION:
-                raise RuntimeError(f"emberserve_amd: _fast.so is not built or has ABI version {fast.ABI_VERSION} "
-                                   f"(expected {ABI_VERSION}); run `python -m emberserve_amd.build`")
-            fast.bind({name: ctypes.cast(getattr(lib, name), _p).value for name in SIGNATURES})
+            try:
+                from . import _fast
+            except ImportError as e:
+                raise RuntimeError(f"emberserve_amd: _fast.so is not built ({e}); run `python -m "
+                                   "emberserve_amd.build`") from None
+            if _fast.ABI_VERSION != ABI_VERSION:
+                raise RuntimeError(f"emberserve_amd: _fast.so has ABI version {_fast.ABI_VERSION}, expected "
+                                   f"{ABI_VERSION}; rebuild it")
+            _fast.bind({name: ctypes.cast(getattr(lib, name), _p).value for name in SIGNATURES})
+            fast.__dict__.update({k: v for k, v in vars(_fast).items() if not k.startswith("__")})
             _lib = lib
         return lib
 

@@ -5,6 +5,9 @@ the others (which the wrappers convert, refuse or run eagerly)."""
 
 from __future__ import annotations
 
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -42,6 +45,14 @@ def test_every_function_declines_cpu_tensors():
     assert fast.paged_decode(q, cache, cache, pos.int()[:, None], pos.int(), 1.0, None) is None
     assert fast.mla_decode(q, q, cache[..., 0, :], pos.int()[:, None], pos.int(), 1.0, None) is None
     assert fast.rmsnorm("x", None, 1e-6) is None and fast.rmsnorm(x) is None  # no tensors, no such arguments
+
+
+def test_extension_is_imported_by_load():
+    """A process may import the package before anything is built: the extension comes with load()."""
+    code = ("import sys, emberserve_amd; from emberserve_amd import _lib\n"
+            "assert 'emberserve_amd._fast' not in sys.modules and _lib.fast.rmsnorm(1) is None\n"
+            "_lib.load(); assert 'rmsnorm' in vars(_lib.fast)")
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=300)
 
 
 gpu = pytest.mark.gpu
