@@ -403,7 +403,8 @@ k_gate_up_silu_gemm(GemmArgs a) {
 
 // ---------------------------------------------------------------- packed weight, dense
 //
-// k_gate_up_silu_gemm_frag: the dense GEMM over the decode kernels' packed weight. Every 1 KiB
+// k_gate_up_silu_gemm_frag: the GEMM over the decode kernels' packed weight (dense, or an
+// expert's: MOE, token tiles of 64 or 128 assignments). Every 1 KiB
 // block of the packed layout is one MFMA operand fragment, so the weights go from memory
 // straight to registers, one contiguous KiB per load, and only x passes through LDS. With
 // both operands in LDS (k_gate_up_silu_gemm) a 256 x (128 + 128) tile reads 192 KB and writes
@@ -432,6 +433,11 @@ k_gate_up_silu_gemm(GemmArgs a) {
 // silu_and_mul): Qwen3-8B 64 tokens 68 -> 41 | 45, 128: 69 -> 46 | 50, 200: 70 -> 60 | 63, 512:
 // 115 -> 90 | 92, 8192: 1450 -> 1320 | 1205; Qwen2.5-7B 64: 78 -> 52 | 62, 256: 100 -> 76 | 80,
 // 600: 217 -> 174 | 171; Qwen2.5-0.5B 130: 21 -> 12.3 | 12.6, 2000: 62 -> 45 | 70.
+// Routed experts (H 2048, I 1408, 64 experts, top-6; without the alignment): 128-row blocks
+// at 512 tokens 147 -> 144, 2048: 258 -> 251, 8192: 767 -> 715; 64-row ones at 128 tokens 129,
+// 256: 133 (128-row ones 143 before). 256-row blocks stay with k_gate_up_silu_gemm: their
+// weights, shared by few blocks, would cross the vector memory path twice (4099 tokens 367,
+// here 388).
 __device__ __forceinline__ auto gemm_rsrc(const void* p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, -1, kBufferWord3);
@@ -494,7 +500,7 @@ struct SlabWalk {
 template <int V>
 using IntC = std::integral_constant<int, V>;
 
-template <typename T, int BM, int CG, int CW>
+template <typename T, int BM, int CG, int CW, bool MOE>
 __global__ void __launch_bounds__(128 * CG, (2 * CG + 3) / 4)
 k_gate_up_silu_gemm_frag(GemmArgs a) {
   using M = GemmMfma<T>;
@@ -505,7 +511,7 @@ k_gate_up_silu_gemm_frag(GemmArgs a) {
   constexpr int NX = TW / 16;            // x fragments per 32 k
   constexpr int NC = CW / 16;            // 16-column tiles per wave
   constexpr int NF = 2 * NC;             // weight fragments per 32 k
-  static_assert(BM % 64 == 0 && (CW == 16 || CW == 32) && 64 % CW == 0, "a wave's columns lie in one slab");
+  static_assert(BM % 32 == 0 && (CW == 16 || CW == 32) && 64 % CW == 0, "a wave's columns lie in one slab");
   constexpr int XREG = BM * kGemmRowB;   // one x stage (64 k)
   constexpr int NBUF = 4;                // x ring: two stages of loads in flight
   constexpr int XI = BM / 8;             // x load instructions (8 rows) per stage
@@ -523,14 +529,25 @@ k_gate_up_silu_gemm_frag(GemmArgs a) {
   const int n = lane & 15, g = lane >> 4;
 
   // XCD-aware tile order, then GROUP_M token tiles per band of column tiles
-  const int mtiles = (a.T + BM - 1) / BM;
+  int mtiles = (a.T + BM - 1) / BM;
   const int ntiles = (a.I + BNG - 1) / BNG;
   int pid = blockIdx.x;
+  int nb = gridDim.x;
+  if (MOE) {  // only the used blocks share out the chip (see k_gate_up_silu_gemm)
+    int used = 0;
+    for (int i0 = 0; i0 < mtiles; i0 += kWave) {
+      const int i = i0 + lane;
+      const bool u = i < mtiles && a.block_expert[i] < a.E;
+      used += __builtin_popcountll(__ballot(u));
+    }
+    mtiles = used;
+    nb = used * ntiles;
+  }
   {
-    const int nb = gridDim.x;
     const int per = (nb + 7) / 8;
     const int xcd = pid % 8, idx = pid / 8;
     const int full = nb % 8 == 0 ? 8 : nb % 8;
+    if (MOE && idx >= (xcd < full ? per : per - 1)) return;
     pid = xcd < full ? xcd * per + idx : full * per + (xcd - full) * (per - 1) + idx;
   }
   constexpr int GM = EMBER_GEMM_GROUP_M;
@@ -543,7 +560,12 @@ k_gate_up_silu_gemm_frag(GemmArgs a) {
 
   // x: byte offsets of this lane's 16 bytes from the tile's first row (padded tokens: the last
   // real row); instruction ins moves rows 8 ins .. 8 ins + 7
-  const T* X = static_cast<const T*>(a.x) + static_cast<int64_t>(m0) * a.xs;
+  const T* X = static_cast<const T*>(a.x) + (MOE ? 0 : static_cast<int64_t>(m0) * a.xs);
+  int64_t expert = 0;
+  if (MOE) {
+    expert = a.block_expert[mt];  // uniform
+    if (expert < 0 || expert >= a.E) return;
+  }
   const auto xrsrc = gemm_rsrc(X);
   const int nd = a.H / 64;
   int src[XL], dst[XL];
@@ -552,7 +574,16 @@ k_gate_up_silu_gemm_frag(GemmArgs a) {
     const int ins = min(XL * w + i, XI - 1);
     const int xr = 8 * ins + (lane >> 3);
     const int c = (lane & 7) ^ (xr & 7);
-    src[i] = static_cast<int>((min(xr, a.T - 1 - m0) * a.xs + 8 * c) * static_cast<int64_t>(sizeof(T)));
+    int64_t xrow = min(xr, a.T - 1 - m0);
+    if (MOE) {  // padding assignments read token 0 and store nothing
+      const int id = a.sorted_ids[m0 + xr];
+      xrow = id >= 0 && id < a.num_valid ? id / a.top_k : 0;
+      if (xrow >= a.ntok) {  // a corrupt layout: flag it, read token 0 (the row is stored)
+        atomicOr(a.err, EMBER_ERR_ROW_INDEX);
+        xrow = 0;
+      }
+    }
+    src[i] = static_cast<int>((xrow * a.xs + 8 * c) * static_cast<int64_t>(sizeof(T)));
     dst[i] = ins * 1024;
   }
   auto issue_x = [&](int d) __attribute__((always_inline)) {
@@ -563,14 +594,24 @@ k_gate_up_silu_gemm_frag(GemmArgs a) {
   // weights: the wave's first column, the last real ones past I (nothing of those is stored)
   const int c0 = n0 + CW * cg;
   const int cw = min(c0, a.I - CW);
-  const unsigned char* W = static_cast<const unsigned char*>(a.w) + ((cw % 64) / 16) * 2048;
+  const unsigned char* W = static_cast<const unsigned char*>(a.w) + ((cw % 64) / 16) * 2048 +
+                           expert * a.wes * static_cast<int64_t>(sizeof(T));
   const uint32_t lane16 = 16u * lane;
+  // The weights' unit of each stage: the dense packing's place is walked, an expert's units are
+  // k-major (unit j slabs + slab).
   SlabWalk walk;
-  walk.init(cw / 64, nd, a.pk_total, a.pk_G);
-  int64_t unit = 0;  // byte offset of the current unit
+  if (!MOE) walk.init(cw / 64, nd, a.pk_total, a.pk_G);
+  const int64_t kstep = MOE ? static_cast<int64_t>(a.I / 64) * 16384 : 0;
+  int64_t unit = MOE ? static_cast<int64_t>(cw / 64) * 16384 - kstep : 0;  // byte offset of the current unit
+  int left = nd;
   auto next_unit = [&]() __attribute__((always_inline)) {
-    unit = static_cast<int64_t>(walk.pos()) * 16384;
-    walk.advance();
+    if (MOE) {  // past the last stage it stays there
+      unit += left > 0 ? kstep : 0;
+      --left;
+    } else {
+      unit = static_cast<int64_t>(walk.pos()) * 16384;
+      walk.advance();
+    }
   };
   V8 fw[WR][NF];
   auto load_w = [&](V8 (&f)[NF], int half) __attribute__((always_inline)) {
@@ -646,8 +687,13 @@ k_gate_up_silu_gemm_frag(GemmArgs a) {
   T* out = static_cast<T*>(a.out);
 #pragma unroll
   for (int u = 0; u < NX; ++u) {
-    const int tok = m0 + TW * q + 16 * u + n;
-    if (tok < a.T) {
+    int tok = m0 + TW * q + 16 * u + n;
+    bool real = tok < a.T;
+    if (MOE) {  // the assignment's own output row
+      tok = a.sorted_ids[tok];
+      real = tok >= 0 && tok < a.num_valid;
+    }
+    if (real) {
 #pragma unroll
       for (int t = 0; t < NC; ++t) {
         Pack<T, 4> o;
@@ -664,11 +710,11 @@ k_gate_up_silu_gemm_frag(GemmArgs a) {
   }
 }
 
-template <typename T, int BM, int CG, int CW>
+template <typename T, int BM, int CG, int CW, bool MOE = false>
 int launch_frag(const GemmArgs& a, hipStream_t st) {
   const int64_t grid = cdiv(a.T, BM) * cdiv(a.I, CG * CW);
   if (grid > 0x7fffffffLL) return EMBER_EINVAL;
-  k_gate_up_silu_gemm_frag<T, BM, CG, CW><<<dim3(static_cast<uint32_t>(grid)), dim3(128 * CG), 0, st>>>(a);
+  k_gate_up_silu_gemm_frag<T, BM, CG, CW, MOE><<<dim3(static_cast<uint32_t>(grid)), dim3(128 * CG), 0, st>>>(a);
   return launch_status();
 }
 
@@ -854,19 +900,22 @@ extern "C" int ember_gate_up_silu_gemm_packed_auto(const void* x, int64_t x_row_
                                  out_row_stride, stream);
 }
 
-extern "C" int ember_moe_gate_up_silu_gemm_packed(const void* x, int64_t x_row_stride, int64_t num_tokens,
-                                                  const void* packed, int dtype, int64_t num_experts, int64_t hidden,
-                                                  int64_t inter, const int32_t* sorted_ids,
-                                                  const int32_t* block_expert, int64_t num_blocks, int64_t block_rows,
-                                                  int64_t num_valid, int64_t top_k, int64_t column_tile, void* out,
-                                                  int64_t out_row_stride, void* stream) {
-  using namespace ember;
+namespace ember {
+namespace {
+
+// The packed experts' entry points' body; `rows64` admits the 64-row blocks.
+int moe_gemm_packed_core(const void* x, int64_t x_row_stride, int64_t num_tokens, const void* packed, int dtype,
+                         int64_t num_experts, int64_t hidden, int64_t inter, const int32_t* sorted_ids,
+                         const int32_t* block_expert, int64_t num_blocks, int64_t block_rows, int64_t num_valid,
+                         int64_t top_k, int64_t column_tile, bool rows64, void* out, int64_t out_row_stride,
+                         void* stream) {
   if (num_blocks == 0 || num_valid == 0) return EMBER_OK;
   if (num_blocks < 0 || num_valid < 0 || num_tokens < 1 || top_k < 1 || num_experts < 1 || num_blocks > (1 << 22) ||
       num_valid > INT32_MAX / 2 || num_tokens > INT32_MAX || hidden < 64 || hidden % 64 != 0 ||
       hidden > (int64_t(1) << 20) || inter < 64 || inter > (int64_t(1) << 28))
     return EMBER_EINVAL;
-  const bool shape = (block_rows == 256 && (column_tile == 64 || column_tile == 128)) ||
+  const bool shape = (rows64 && block_rows == 64 && column_tile == 128) ||
+                     (block_rows == 256 && (column_tile == 64 || column_tile == 128)) ||
                      (block_rows == 128 && column_tile == 128);
   if (!shape || inter % column_tile != 0) return EMBER_EINVAL;
   if (dtype != EMBER_F16 && dtype != EMBER_BF16) return EMBER_EINVAL;
@@ -880,13 +929,45 @@ extern "C" int ember_moe_gate_up_silu_gemm_packed(const void* x, int64_t x_row_s
              static_cast<int>(num_valid), static_cast<int>(top_k), static_cast<int>(num_experts),
              static_cast<int>(num_tokens), 2 * inter * hidden, device_error_word(), 0, 1};
   if (a.err == nullptr) return EMBER_ENODEV;
+  // the frag kernel addresses x rows by 32-bit offsets
+  const bool frag = num_tokens * x_row_stride < (int64_t(1) << 29);
+  if (block_rows == 64 && !frag) return EMBER_ETOOBIG;
   const hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == EMBER_F16) {
+    if (block_rows == 128 && frag) return launch_frag<_Float16, 128, 4, 32, true>(a, st);
+    if (block_rows == 64) return launch_frag<_Float16, 64, 4, 32, true>(a, st);
     if (block_rows == 128) return launch_gemm<_Float16, 128, 128, true, true>(a, st);
     return column_tile == 64 ? launch_gemm<_Float16, 64, 256, true, true>(a, st)
                              : launch_gemm<_Float16, 128, 256, true, true>(a, st);
   }
+  if (block_rows == 128 && frag) return launch_frag<__bf16, 128, 4, 32, true>(a, st);
+  if (block_rows == 64) return launch_frag<__bf16, 64, 4, 32, true>(a, st);
   if (block_rows == 128) return launch_gemm<__bf16, 128, 128, true, true>(a, st);
   return column_tile == 64 ? launch_gemm<__bf16, 64, 256, true, true>(a, st)
                            : launch_gemm<__bf16, 128, 256, true, true>(a, st);
+}
+
+}  // namespace
+}  // namespace ember
+
+extern "C" int ember_moe_gate_up_silu_gemm_packed(const void* x, int64_t x_row_stride, int64_t num_tokens,
+                                                  const void* packed, int dtype, int64_t num_experts, int64_t hidden,
+                                                  int64_t inter, const int32_t* sorted_ids,
+                                                  const int32_t* block_expert, int64_t num_blocks, int64_t block_rows,
+                                                  int64_t num_valid, int64_t top_k, int64_t column_tile, void* out,
+                                                  int64_t out_row_stride, void* stream) {
+  return ember::moe_gemm_packed_core(x, x_row_stride, num_tokens, packed, dtype, num_experts, hidden, inter, sorted_ids,
+                                     block_expert, num_blocks, block_rows, num_valid, top_k, column_tile, false, out,
+                                     out_row_stride, stream);
+}
+
+extern "C" int ember_moe_gate_up_silu_gemm_packed_rows64(const void* x, int64_t x_row_stride, int64_t num_tokens,
+                                                         const void* packed, int dtype, int64_t num_experts,
+                                                         int64_t hidden, int64_t inter, const int32_t* sorted_ids,
+                                                         const int32_t* block_expert, int64_t num_blocks,
+                                                         int64_t num_valid, int64_t top_k, void* out,
+                                                         int64_t out_row_stride, void* stream) {
+  return ember::moe_gemm_packed_core(x, x_row_stride, num_tokens, packed, dtype, num_experts, hidden, inter, sorted_ids,
+                                     block_expert, num_blocks, 64, num_valid, top_k, 128, true, out, out_row_stride,
+                                     stream);
 }

@@ -263,16 +263,43 @@ def moe_gate_up_silu(x: Tensor, w_gate_up: Tensor, sorted_ids: Tensor, block_exp
 
 
 GEMM_BLOCK_M = 256  # rows per block of the prefill GEMM's layout (its token tile)
-# fused_moe_gate_up: the GEMM from GEMM_FROM assignments (128-row blocks below
-# GEMM_WIDE_FROM, 256-row ones from there), the packed 16-block kernel up to
-# PACKED_MAX_ASSIGNMENTS. Measured at Moonlight's geometry (bf16, µs, alignment included;
-# row kernel at its default splits | GEMM 256 x 128 | GEMM 128 x 128): 1536 assignments
-# 226 | 259 | 200, 3072: 291 | 292 | 204, 6144: 499 | 282 | 243, 12288: 840 | 341 | 294,
-# 49152: 2722 | 688 | 736. The packed kernel: 384 assignments 115 against the row
-# kernel's 136; 1536: 228 against 205.
+# fused_moe_gate_up's kernels by routed assignments (A, per expert: a). Measured with
+# std-0.3 expert biases, bf16, weights alternating, µs with the alignment (64 experts top-6 H 2048
+# I 1408, A = 6 tokens | 128 experts top-8 H 2048 I 768 | 8 experts top-2 H 4096 I 3584):
+# - 64-row blocks over packed experts from a = ROWS64_PER_EXPERT where the experts' tiles fill the
+#   chip, or from A = GEMM_FROM, below ROWS128_PER_EXPERT. 16-block kernels (packed; row past
+#   PACKED_MAX_ASSIGNMENTS) | 64-row blocks: 96 tokens 127 | 136, 128: 149 | 136, 192: 182 | 140; E 128,
+#   128 tokens 145 | 147; E 8, 64 tokens 114 | 83. 128-row | 64-row blocks: 256 tokens 150 | 143, 384:
+#   158 | 147, 512: 161 | 167; E 128, 256 tokens 162 | 152, 512: 168 | 176.
+# - the 128-row GEMM from A = GEMM_FROM, or from GEMM_PER_EXPERT each where the experts' tiles fill the
+#   chip: row kernel | 128-row GEMM, 128 tokens 157 | 161, 192: 182 | 169, 256: 202 | 170; E 8,
+#   64 tokens 119 | 93, 128: 138 | 98, 384: 305 | 150.
+# - 256-row blocks from A = GEMM_WIDE_FROM, or from GEMM_WIDE_PER_EXPERT each and A =
+#   GEMM_WIDE_FILL: 128-row | 256-row blocks, packed, means of five routings, 1536 tokens 228 | 227
+#   (from -13% to +12% each), 1800: 242 | 246, 2048: 267 | 251, 3072: 342 | 315, one at 4099: 407 |
+#   372; E 128, 2048 tokens (a = 128) 232 | 243, 2560: 264 | 247, 4096: 343 | 319; E 8, 768 tokens
+#   (A = 1536) 157 | 200.
 GEMM_FROM = 1536
+GEMM_PER_EXPERT = 16
 GEMM_WIDE_FROM = 24576
+GEMM_WIDE_FILL = 12288
+GEMM_WIDE_PER_EXPERT = 192
+ROWS64_PER_EXPERT = 10
+ROWS128_PER_EXPERT = 32
 PACKED_MAX_ASSIGNMENTS = 768
+
+
+def moe_gemm_block_rows(num_assignments: int, num_experts: int, inter: int, cus: int, packed: bool) -> int:
+    """Rows per block of the GEMM that `fused_moe_gate_up` runs over 128-column tiles: 64 (packed
+    experts only), 128 or 256; 0 for the 16-block kernels."""
+    a, e = num_assignments, num_experts
+    fills = 8 * e * (inter // 128) >= 7 * cus  # measured down to 224 tiles on 256 CUs
+    if packed and a < ROWS128_PER_EXPERT * e and (a >= GEMM_FROM or (fills and a >= ROWS64_PER_EXPERT * e)):
+        return 64
+    if a < GEMM_FROM and not (fills and a >= GEMM_PER_EXPERT * e):
+        return 0
+    wide = a >= GEMM_WIDE_FROM or (a >= GEMM_WIDE_FILL and a >= GEMM_WIDE_PER_EXPERT * e)
+    return 256 if wide else 128
 
 
 def moe_gate_up_silu_gemm(x: Tensor, w_gate_up: Tensor | None, topk_ids: Tensor, *, column_tile: int = 128,
@@ -330,6 +357,22 @@ def moe_gate_up_silu_gemm(x: Tensor, w_gate_up: Tensor | None, topk_ids: Tensor,
     return out
 
 
+def _moe_gemm_rows64(x: Tensor, topk_ids: Tensor, packed: PackedExperts) -> Tensor:
+    """`moe_gate_up_silu_gemm` over the packed experts and 64-row blocks
+    (`ember_moe_gate_up_silu_gemm_packed_rows64`; operands checked by the caller)."""
+    _require_device("moe_gate_up_silu_gemm", x, packed.packed, topk_ids)
+    n, k = topk_ids.shape
+    sorted_ids, block_expert, num_valid = moe_align(topk_ids, packed.num_experts, 64)
+    out = torch.empty((num_valid, packed.inter), dtype=x.dtype, device=x.device)
+    _launch("ember_moe_gate_up_silu_gemm_packed_rows64", _lib.load().ember_moe_gate_up_silu_gemm_packed_rows64,
+            x.device, x.data_ptr(), x.stride(0), x.shape[0], packed.packed.data_ptr(), _lib.dtype_tag(x.dtype),
+            packed.num_experts, packed.hidden, packed.inter, sorted_ids.data_ptr(), block_expert.data_ptr(),
+            block_expert.numel(), num_valid, k, out.data_ptr(), out.stride(0))
+    if _check_indices() and _lib.read_errors(clear=True) & _lib.ERR_ROW_INDEX:
+        raise IndexError("emberserve_amd.moe_gate_up_silu_gemm: assignment id past the token rows")
+    return out
+
+
 def moe_gate_up_silu_direct(x: Tensor, topk_ids: Tensor, packed: PackedExperts, *,
                             half_slabs: bool = False) -> Tensor:
     """act [N * k, I] straight from the routing ids, without moe_align
@@ -361,10 +404,10 @@ def fused_moe_gate_up(x: Tensor, topk_ids: Tensor, w_gate_up: Tensor, *, num_spl
                       packed: PackedExperts | None = None) -> Tensor:
     """The routed experts' activations [N * k, I] in assignment order (the `act` of
     moe_triton.py:340): up to DIRECT_MAX_TOKENS tokens over a packed weight straight from the
-    routing ids; from
-    GEMM_FROM assignments the prefill GEMM (`moe_gate_up_silu_gemm`); otherwise moe_align +
-    the 16-block kernel (`moe_gate_up_silu`, packed up to PACKED_MAX_ASSIGNMENTS). Every
-    path gives the same bits as the 16-block kernel at one k split."""
+    routing ids; then the prefill GEMM (`moe_gate_up_silu_gemm`) where `moe_gemm_block_rows`
+    gives it blocks; otherwise moe_align + the 16-block kernel (`moe_gate_up_silu`, packed up to
+    PACKED_MAX_ASSIGNMENTS or ROWS64_PER_EXPERT each). Every path gives the same bits as the
+    16-block kernel at one k split."""
     aligned = x.is_cuda and fused_enabled(x) and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
     n, k = topk_ids.shape
     if (packed is not None and num_splits is None and n <= DIRECT_MAX_TOKENS and n * k <= DIRECT_MAX_ASSIGNMENTS
@@ -373,17 +416,29 @@ def fused_moe_gate_up(x: Tensor, topk_ids: Tensor, w_gate_up: Tensor, *, num_spl
         half = moe_direct_half_slabs(n * k, packed.num_experts, packed.inter, x.device)
         return moe_gate_up_silu_direct(x, topk_ids, packed, half_slabs=half)
     E, two_i, H = w_gate_up.shape
-    if (num_splits is None and n * k >= GEMM_FROM and aligned and x.dtype == w_gate_up.dtype
-            and x.dtype in SUPPORTED_DTYPES and H % 64 == 0 and (two_i // 2) % 64 == 0
+    inter = two_i // 2
+    a = n * k
+    fits = packed is not None and (packed.num_experts, packed.hidden, packed.inter, packed.dtype,
+                                   packed.device) == (E, H, inter, x.dtype, x.device)
+    if (num_splits is None and a > 0 and aligned and x.dtype == w_gate_up.dtype
+            and x.dtype in SUPPORTED_DTYPES and H % 64 == 0 and inter % 64 == 0
             and w_gate_up.stride(2) == 1 and w_gate_up.stride(1) % 8 == 0 and w_gate_up.stride(0) % 8 == 0
             and w_gate_up.data_ptr() % 16 == 0):
         # over the packed experts when there are (contiguous units; the same bits)
-        if (two_i // 2) % 128 == 0:
-            rows = 128 if n * k < GEMM_WIDE_FROM else 256
-            return moe_gate_up_silu_gemm(x, w_gate_up, topk_ids, column_tile=128, block_rows=rows, packed=packed)
-        return moe_gate_up_silu_gemm(x, w_gate_up, topk_ids, column_tile=64, block_rows=256, packed=packed)
-    if packed is not None and n * k > PACKED_MAX_ASSIGNMENTS:
-        packed = None  # the row kernel is faster there (see PACKED_MAX_ASSIGNMENTS)
+        if inter % 128 == 0:
+            # operands that the 16-block kernels refuse reach them below GEMM_FROM, and are refused
+            match = (x.dim() == 2 and x.shape[1] == H and n <= x.shape[0] and two_i % 2 == 0
+                     and w_gate_up.device == x.device)
+            rows = moe_gemm_block_rows(a, E, inter, num_sms(x.device),  # 64 rows: 32-bit offsets into x
+                                       fits and match and x.shape[0] * x.stride(0) < 2 ** 29)
+            if rows == 64:
+                return _moe_gemm_rows64(x, topk_ids, packed)
+            if rows and (a >= GEMM_FROM or (match and (packed is None or fits))):
+                return moe_gate_up_silu_gemm(x, w_gate_up, topk_ids, column_tile=128, block_rows=rows, packed=packed)
+        elif a >= GEMM_FROM:
+            return moe_gate_up_silu_gemm(x, w_gate_up, topk_ids, column_tile=64, block_rows=256, packed=packed)
+    if a > max(PACKED_MAX_ASSIGNMENTS, ROWS64_PER_EXPERT * E if fits else 0):
+        packed = None  # the row kernel is faster there
     sorted_ids, block_expert, num_valid = moe_align(topk_ids, E)
     return moe_gate_up_silu(x, w_gate_up, sorted_ids, block_expert, num_valid, k,
                             num_splits=num_splits, packed=packed)

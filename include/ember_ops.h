@@ -546,6 +546,15 @@ int ember_moe_gate_up_silu_gemm_packed(const void* x, int64_t x_row_stride, int6
                                        int64_t block_rows, int64_t num_valid, int64_t top_k, int64_t column_tile,
                                        void* out, int64_t out_row_stride, void* stream);
 
+/* ember_moe_gate_up_silu_gemm_packed over 64-row blocks (128-column tiles; inter a multiple of
+ * 128), for batches that leave most of a 128-row block empty. EMBER_ETOOBIG from 2^29 elements
+ * of x (num_tokens x_row_stride). The same bits. */
+int ember_moe_gate_up_silu_gemm_packed_rows64(const void* x, int64_t x_row_stride, int64_t num_tokens,
+                                              const void* packed, int dtype, int64_t num_experts, int64_t hidden,
+                                              int64_t inter, const int32_t* sorted_ids, const int32_t* block_expert,
+                                              int64_t num_blocks, int64_t num_valid, int64_t top_k, void* out,
+                                              int64_t out_row_stride, void* stream);
+
 /* Bytes of workspace ember_moe_gate_up_silu needs for num_splits > 1 (0 for one split), -1
  * for invalid arguments: fp32 partials [num_splits][num_valid][2 inter] and one uint32
  * arrival counter per (block, 64-column slab). */

@@ -317,3 +317,45 @@ def test_prefill_path_graph_replay_with_fresh_ids():
         torch.cuda.synchronize()
         want = fused_moe_gate_up(dx, new.to(DEV), dw)
         assert torch.equal(out, want), rep
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,experts,inter,skew", [(107, 64, 1408, False), (330, 64, 1408, False), (341, 64, 1408, True),
+                                                  (21, 8, 3584, True), (42, 8, 3584, False), (214, 128, 768, False)])
+def test_packed_moe_gemm_64_row_blocks(dtype, n, experts, inter, skew):
+    """fused_moe_gate_up over packed experts at the 64-row blocks' sizes: experts with one, 63, 64
+    and 65 or more assignments (the skew), a padded x row stride, bit-identical to the 16-block row
+    kernel at one k split (both add every product over k in the same order)."""
+    from emberserve_amd.moe import moe_gemm_block_rows
+
+    hidden, k = 320, 6  # five 64-column k steps: an odd count
+    print(f"moe 64-row blocks n={n} E={experts} skew={skew} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(n)
+    x = torch.empty(n, hidden + 8, dtype=dtype, device=DEV)[:, :hidden]
+    x.copy_((torch.randn(n, hidden, generator=g) * 0.5).to(dtype))
+    w = (torch.randn(experts, 2 * inter, hidden, generator=g) * 1.5 / hidden ** 0.5).to(dtype).to(DEV)
+    ids = torch.stack([torch.randperm(experts, generator=g)[:k] for _ in range(n)])
+    if skew:  # experts 0, 1, 2 in the first 63, 64, 65 tokens only
+        ids = torch.stack([torch.randperm(experts - 3, generator=g)[:k] + 3 if experts - 3 >= k
+                           else torch.randint(3, experts, (k,), generator=g) for _ in range(n)])
+        for e, c in enumerate((63, 64, 65)):
+            ids[:c, e] = e
+    ids = ids.to(DEV)
+    assert moe_gemm_block_rows(n * k, experts, inter, 256, True) == 64
+    si, be, nv = moe_align(ids, experts)
+    want = moe_gate_up_silu(x, w, si, be, nv, k, num_splits=1)
+    packed = pack_moe_gate_up_weight(w)
+    assert torch.equal(fused_moe_gate_up(x, ids, w, packed=packed), want)
+    for rows in (128, 256):
+        assert torch.equal(moe_gate_up_silu_gemm(x, None, ids, block_rows=rows, packed=packed), want), rows
+
+
+def test_moe_gemm_block_rows_rule():
+    """The lines of fused_moe_gate_up's choice of blocks, and what stays with the 16-block kernels."""
+    from emberserve_amd.moe import moe_gemm_block_rows as rule
+
+    assert [rule(a, 64, 1408, 256, True) for a in (639, 640, 2047, 2048, 12287, 12288, 24576)] == [
+        0, 64, 64, 128, 128, 256, 256]
+    assert [rule(a, 64, 1408, 256, False) for a in (1023, 1024, 12287, 12288)] == [0, 128, 128, 256]
+    assert [rule(a, 128, 768, 256, True) for a in (1279, 1280, 4096, 24575, 24576)] == [0, 64, 128, 128, 256]
+    assert [rule(a, 8, 1408, 256, p) for a in (160, 1535, 1536) for p in (False, True)] == [0, 0, 0, 0, 128, 128]
