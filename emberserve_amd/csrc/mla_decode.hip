@@ -126,11 +126,12 @@ struct MlaArgs {
   float scale2;                // scale * log2(e)
   int32_t splits;
   int32_t min_tiles;           // MFMA kernels: the least tiles a split takes
-  float* part_m;               // [splits][nseq][nh]
+  float* part_m;               // [splits][nseq][nh]; MFMA kernels: [unit][nh], unit as in mla_plan
   float* part_l;
-  float* part_o;               // [splits][nseq][nh][dl]
+  float* part_o;               // [..][nh][dl]
   uint32_t* counters;          // [nseq][nh] split arrivals (MFMA kernel), zero between launches
   int32_t merge_apart;         // MFMA kernels: publish the partials only, k_mla_merge merges
+  int32_t balance;             // MFMA kernels: split sizes from all contexts (nseq <= 64), see mla_plan
   uint32_t* err;
 };
 
@@ -163,8 +164,7 @@ __device__ __forceinline__ void load_to_lds16(const void* gptr, void* lds_base) 
 #endif
 }
 
-__device__ __forceinline__ int seq_context(const MlaArgs& a, int b) {
-  int c = a.ctx[b];
+__device__ __forceinline__ int seq_context(const MlaArgs& a, int c) {
   const int cap = a.max_blocks * a.block_size;
   if (c < 0 || c > cap) {
     if (threadIdx.x == 0) atomicOr(a.err, EMBER_ERR_DECODE_CTX);
@@ -190,16 +190,66 @@ __device__ __forceinline__ void split_range(int ctx, int splits, int split, int&
   t1 = min(t0 + per, nt);
 }
 
-// How the MFMA kernels cut a context: equal parts of at least min_tiles tiles, so a short
-// context of a ragged batch takes fewer splits than a long one (at least one).
+// Inclusive prefix sum over the wave (all lanes active).
+__device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return v;
+}
+
+// ceil(x / y) for 0 <= x, 0 < y, x + y <= 2^21: the half keeps the quotient further from a whole
+// number than v_rcp_f32's and the product's rounding (1.5 ulp, so under (x + y) 2^-22 / y) moves it.
+__device__ __forceinline__ int small_ceil_div(int x, int y) {
+  return static_cast<int>((static_cast<float>(x + y) - 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(y)));
+}
+
+// How the MFMA kernels cut the contexts into units (workgroups per head chunk), nseq x splits
+// of them at most. Without `balance`, each context into `splits` equal parts of at least
+// min_tiles tiles, so a short context of a ragged batch takes fewer splits than a long one.
+// With it, all into parts of one size, the least of five that fits the units: per =
+// ceil(tiles / (units - k nseq / 4)), k = 0 .. 4 (k = 4 always fits: a context takes at most
+// floor(tiles / per) + 1), so the long contexts of a ragged batch use the units that the short ones
+// leave. Every context takes one unit at least.
 struct SplitPlan {
-  int per;  // tiles per split
-  int n;    // splits that the context takes
+  int first;  // the context's first unit
+  int per;    // tiles per split
+  int n;      // splits that the context takes
 };
-__device__ __forceinline__ SplitPlan split_plan(const MlaArgs& a, int ctx) {
-  const int nt = (ctx + kTile - 1) / kTile;
+struct MlaPlan {
+  int raw, per, n, first;  // balance: lane b's sequence (raw: its context length as given)
+};
+__device__ __forceinline__ MlaPlan mla_plan(const MlaArgs& a) {
+  const int lane = threadIdx.x & (kWave - 1);
+  MlaPlan p{0, 0, 0, 0};
+  if (!a.balance) return p;
+  const bool in = lane < a.nseq;
+  p.raw = in ? a.ctx[lane] : 0;
+  const int nt = (min(max(p.raw, 0), a.max_blocks * a.block_size) + kTile - 1) / kTile;
+  const int total = __builtin_amdgcn_readlane(wave_scan(nt), kWave - 1);
+  const int units = a.nseq * a.splits;
+  for (int k = 0; k <= 4; ++k) {
+    p.per = max(small_ceil_div(total, units - k * a.nseq / 4), a.min_tiles);
+    p.n = in ? max(1, small_ceil_div(nt, p.per)) : 0;
+    const int incl = wave_scan(p.n);
+    p.first = incl - p.n;
+    if (__builtin_amdgcn_readlane(incl, kWave - 1) <= units) break;
+  }
+  return p;
+}
+// Sequence b's part of the plan (b uniform); c: its context length as given.
+__device__ __forceinline__ SplitPlan seq_plan(const MlaArgs& a, const MlaPlan& p, int b, int& c) {
+  if (a.balance) {
+    c = __builtin_amdgcn_readlane(p.raw, b);
+    return {__builtin_amdgcn_readlane(p.first, b), p.per, __builtin_amdgcn_readlane(p.n, b)};
+  }
+  c = a.ctx[b];
+  const int nt = (min(max(c, 0), a.max_blocks * a.block_size) + kTile - 1) / kTile;
   const int per = max((nt + a.splits - 1) / a.splits, a.min_tiles);
-  return {per, max(1, (nt + per - 1) / per)};
+  return {b * a.splits, per, max(1, (nt + per - 1) / per)};
 }
 
 // Workgroup order of the MFMA kernels: units (sequence, split), eight at a time, one per XCD
@@ -207,7 +257,7 @@ __device__ __forceinline__ SplitPlan split_plan(const MlaArgs& a, int ctx) {
 // its XCD, whose L2 then holds their common rows. The units of a group of eight are rotated
 // by the group's number, so that no XCD gets one split number (or every eighth sequence)
 // alone.
-__device__ __forceinline__ void mla_unit(const MlaArgs& a, int& b, int& split, int& hc) {
+__device__ __forceinline__ void mla_unit(const MlaArgs& a, const MlaPlan& p, int& b, int& split, int& hc) {
   const int pid = blockIdx.x + gridDim.x * blockIdx.y;
   const int units8 = (a.nseq * a.splits) & ~7;
   int u;
@@ -222,8 +272,15 @@ __device__ __forceinline__ void mla_unit(const MlaArgs& a, int& b, int& split, i
     u = units8 + r % rem;
     hc = r / rem;
   }
-  split = u % a.splits;
-  b = u / a.splits;
+  u = __builtin_amdgcn_readfirstlane(u);
+  if (a.balance) {  // the last sequence whose units begin at or before u (they begin in order)
+    const int lane = threadIdx.x & (kWave - 1);
+    b = __builtin_popcountll(__ballot(lane < a.nseq && p.first <= u)) - 1;
+    split = u - __builtin_amdgcn_readlane(p.first, b);
+  } else {
+    split = u % a.splits;
+    b = u / a.splits;
+  }
 }
 
 // The end of an MFMA kernel's workgroup: the tile streams merge through LDS, then either
@@ -232,7 +289,7 @@ __device__ __forceinline__ void mla_unit(const MlaArgs& a, int& b, int& split, i
 // wave w of pair w / 2 holds d in [(w % 2) DL / 2, (w % 2 + 1) DL / 2).
 template <typename T, int DL, int NP>
 __device__ __forceinline__ void mla_finish(const MlaArgs& a, unsigned char* lds, float m, float lsum,
-                                           const f32x4 (&o)[DL / 32], int b, int split, int nsplit,
+                                           const f32x4 (&o)[DL / 32], int b, int split, const SplitPlan& plan,
                                            int head0, int nhc, bool poisoned = false) {
   constexpr int NDT = DL / 32;
   struct Combine {
@@ -307,6 +364,7 @@ __device__ __forceinline__ void mla_finish(const MlaArgs& a, unsigned char* lds,
       store_pack<T, 4>(orow + 4 * PARTS * j, r);
     }
   };
+  const int nsplit = plan.n;
   if (nsplit == 1) {
     if (mine) store_out(L);
     return;
@@ -317,8 +375,8 @@ __device__ __forceinline__ void mla_finish(const MlaArgs& a, unsigned char* lds,
   // merge all of them with agent-coherent loads; it returns the counter to zero for the next
   // launch. The workgroup's 16 partial rows of one split are contiguous, so one buffer
   // resource (uniform base, exact size) addresses them.
-  const int64_t stride = int64_t(a.nseq) * a.nh;
-  const int64_t row0 = int64_t(b) * a.nh + head0;  // this chunk's first (sequence, head) row
+  const int64_t row0 = int64_t(plan.first) * a.nh + head0;  // this chunk's first row of split 0's partial
+  const int64_t stride = a.nh;
   if (mine) {
     if (threadIdx.x % PARTS == 0) {
       store_agent(a.part_m + split * stride + row0 + hh, mx);
@@ -334,7 +392,7 @@ __device__ __forceinline__ void mla_finish(const MlaArgs& a, unsigned char* lds,
   __shared__ int is_last;
   __syncthreads();
   if (threadIdx.x == 0) {
-    uint32_t* cnt = a.counters + row0;
+    uint32_t* cnt = a.counters + int64_t(b) * a.nh + head0;
     const uint32_t prev = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     is_last = prev == static_cast<uint32_t>(nsplit - 1);
     if (is_last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -429,13 +487,15 @@ k_mla_mfma(MlaArgs a) {
   const int n = lane & 15;
   const int g = lane >> 4;
 
+  const MlaPlan all = mla_plan(a);
   int b, split, hc;
-  mla_unit(a, b, split, hc);
+  mla_unit(a, all, b, split, hc);
   const int head0 = hc * 16;
   const int nhc = min(16, a.nh - head0);
 
-  const int ctx = seq_context(a, b);
-  const SplitPlan plan = split_plan(a, ctx);
+  int raw;
+  const SplitPlan plan = seq_plan(a, all, b, raw);
+  const int ctx = seq_context(a, raw);
   if (split >= plan.n) return;
   const int t0 = split * plan.per;
   const int t1 = min(t0 + plan.per, (ctx + kTile - 1) / kTile);
@@ -671,7 +731,7 @@ k_mla_mfma(MlaArgs a) {
   // the output rows of this workgroup (or the merge of its split) come out NaN instead of a
   // plausible wrong value, next to the EMBER_ERR_SYNC bit.
   if (!sync_ok) poison_state(m, lsum, o);
-  mla_finish<T, DL, NP>(a, lds, m, lsum, o, b, split, plan.n, head0, nhc, !sync_ok);
+  mla_finish<T, DL, NP>(a, lds, m, lsum, o, b, split, plan, head0, nhc, !sync_ok);
 }
 
 // k_mla_lds: the small-grid form of k_mla_mfma (same work split: two wave pairs per
@@ -712,13 +772,15 @@ k_mla_lds(MlaArgs a) {
   const int n = lane & 15;
   const int g = lane >> 4;
 
+  const MlaPlan all = mla_plan(a);
   int b, split, hc;
-  mla_unit(a, b, split, hc);
+  mla_unit(a, all, b, split, hc);
   const int head0 = hc * 16;
   const int nhc = min(16, a.nh - head0);
 
-  const int ctx = seq_context(a, b);
-  const SplitPlan plan = split_plan(a, ctx);
+  int raw;
+  const SplitPlan plan = seq_plan(a, all, b, raw);
+  const int ctx = seq_context(a, raw);
   if (split >= plan.n) return;
   const int t0 = split * plan.per;
   const int t1 = min(t0 + plan.per, (ctx + kTile - 1) / kTile);
@@ -927,7 +989,7 @@ k_mla_lds(MlaArgs a) {
   // the output rows of this workgroup (or the merge of its split) come out NaN instead of a
   // plausible wrong value, next to the EMBER_ERR_SYNC bit.
   if (!sync_ok) poison_state(m, lsum, o);
-  mla_finish<T, DL, NP>(a, lds, m, lsum, o, b, split, plan.n, head0, nhc, !sync_ok);
+  mla_finish<T, DL, NP>(a, lds, m, lsum, o, b, split, plan, head0, nhc, !sync_ok);
 }
 
 constexpr int kAnyMaxD = 1024;          // DL + DR of the fp32 kernel
@@ -946,7 +1008,7 @@ k_mla_any(MlaArgs a) {
   const int split = blockIdx.y;
   const int DL = a.dl;
   const int D = a.dl + a.dr;
-  const int ctx = seq_context(a, b);
+  const int ctx = seq_context(a, a.ctx[b]);
   int t0, t1;
   split_range(ctx, a.splits, split, t0, t1);
   const int kbeg = t0 * kTile;
@@ -1067,15 +1129,18 @@ __global__ void __launch_bounds__(kWave)
 k_mla_merge(MlaArgs a) {
   constexpr int TPR = DL / 4;
   constexpr int kChunk = 8;
+  static_assert(TPR % kWave == 0, "a wave's row is uniform");
   const int t = blockIdx.x * kWave + threadIdx.x;
-  const int row = t / TPR;  // sequence * nh + head
+  const int row = __builtin_amdgcn_readfirstlane(t / TPR);  // sequence * nh + head
   if (row >= a.nseq * a.nh) return;
   const int d = (t % TPR) * 4;
-  const int64_t stride = int64_t(a.nseq) * a.nh;
   const int b = row / a.nh;
-  const int cap = a.max_blocks * a.block_size;
-  const int nsplit = split_plan(a, min(max(a.ctx[b], 0), cap)).n;
+  int raw;
+  const SplitPlan plan = seq_plan(a, mla_plan(a), b, raw);
+  const int nsplit = plan.n;
   if (nsplit == 1) return;  // its only split wrote the output rows
+  const int64_t stride = a.nh;
+  const int64_t row0 = int64_t(plan.first) * a.nh + (row - b * a.nh);
   float gm = -INFINITY, gl = 0.f;
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int c0 = 0; c0 < nsplit; c0 += kChunk) {
@@ -1087,7 +1152,7 @@ k_mla_merge(MlaArgs a) {
       ls[u] = 0.f;
       v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (c0 + u < nsplit) {
-        const int64_t r = (c0 + u) * stride + row;
+        const int64_t r = (c0 + u) * stride + row0;
         ms[u] = a.part_m[r];
         ls[u] = a.part_l[r];
         // part_o starts 8 bytes past a 16-byte boundary when splits x rows is odd
@@ -1256,6 +1321,13 @@ int ember_mla_decode(const void* q_c, int64_t qc_seq_stride, int64_t qc_head_str
                                 max_blocks * block_size >= num_splits * 2 * kMlaPairsSmall * kTile);
     a.min_tiles = small ? 1 : kMlaMinTiles;
     a.merge_apart = num_splits >= kMlaMergeApart ? 1 : 0;
+    // Splits of one size (mla_plan) from 512 keys of table width a split. Ragged contexts (uniform
+    // up to the width), bf16, equal parts | one size: 32 x 4096 28.0 -> 25.8 us, 32 x 8192 42.9 ->
+    // 34.8, 48 x 4096 36.0 -> 29.8, 64 x 8192 71.1 -> 58.1, 16 x 8192 29.0 -> 27.8; contexts of one
+    // length pay the plan, 32 x 4096 34.0 -> 34.3, 16 x 8192 33.8 -> 34.7. Below: 16 x 4096 20.4 -> 22.1.
+    // (The other bounds: one lane per sequence, and the sums of mla_plan's divisions.)
+    a.balance = a.merge_apart && num_seqs > 1 && num_seqs <= kWave && max_blocks * block_size >= num_splits * 512 &&
+                num_seqs * (max_blocks * block_size / kTile + 1 + num_splits) <= (1 << 20);
     if (q_dtype == EMBER_F16)
       launch_mfma<_Float16>(a, grid, small, four, st);
     else

@@ -128,6 +128,45 @@ def test_ragged_full_grids_with_stale_rows(dtype, batch, heads, splits):
     assert _lib.read_errors() == 0
 
 
+@pytest.mark.parametrize("lens,heads,splits", [
+    ("ragged", 16, 4), ("ragged", 20, 5), ("equal", 16, 4), ("one long", 16, 8), ("empty", 16, 4), ("all short", 16, 4)])
+@pytest.mark.parametrize("batch", [2, 33, 64])
+def test_splits_of_one_size_over_the_batch(batch, lens, heads, splits):
+    """Wide tables (512 keys a split): the splits' size comes from all contexts. Uneven and equal
+    contexts, one context that takes nearly every unit, empty ones, and contexts under the least
+    split; captured once and replayed with the contexts reversed, then restored."""
+    _say(f"mla one-size splits B={batch} {lens} H={heads} splits {splits}")
+    g = torch.Generator().manual_seed(batch)
+    wide = 64 * splits // 2  # 16-key blocks: 512 keys of width a split
+    ctx_lens = {"ragged": torch.randint(1, 700, (batch,), generator=g).tolist(), "equal": [320] * batch,
+                "one long": [1] * (batch - 1) + [16 * wide], "empty": [0] * (batch - 1) + [513],
+                "all short": [33] * batch}[lens]
+    q, lat, bt, ctx = gen.mla_decode_inputs(ctx_lens, heads, DL, DR, 16, torch.bfloat16, seed=batch, table_width=wide)
+    dq, dlat, dbt, dctx = (t.to(DEV) for t in (q, lat, bt, ctx))
+    out = torch.empty(batch, heads, DL, dtype=torch.bfloat16, device=DEV)
+
+    def check(order):
+        rows = [b for b in range(batch) if ctx_lens[order[b]]]
+        src = [order[b] for b in rows]
+        _check(out[rows], q[rows][..., :DL], q[rows][..., DL:], lat, bt[src], ctx[src], SCALE, DL, True, f"{lens}")
+
+    same, rev = list(range(batch)), list(range(batch))[::-1]
+    mla_decode(dq, dlat, dbt, dctx, SCALE, DL, num_splits=splits, out=out)
+    check(same)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        mla_decode(dq, dlat, dbt, dctx, SCALE, DL, num_splits=splits, out=out)
+    for order in (rev, same):
+        dbt.copy_(bt[order].to(DEV))
+        dctx.copy_(ctx[order].to(DEV))
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        check(order)
+    assert _lib.read_errors() == 0
+
+
 def test_long_contexts_cross_block_id_windows():
     """Contexts of 9000 and 5000 keys at one and two splits: each wave walks 40-71 tiles,
     crossing the 32-tile windows of prefetched block ids; block size 32 (two halves per
