@@ -13,8 +13,8 @@
 //     the tile and WC = BNG BM / 512 columns of both the gate and the up half, so it holds
 //     (2 WC / 16) x 4 accumulator tiles of 16 x 16;
 //   * the tile's operands stream through an LDS ring of "double stages" of 64 k (three for
-//     the 256 x 64 and 128 x 128 tiles; for 256 x 96 and 256 x 128, where three would not fit, separate
-//     rings of three weight and two x buffers, 160 KiB: 94 instead of 102 us for Qwen3-8B
+//     the 256 x 64 and 128 x 128 tiles; for 256 x 96 and 256 x 128, where three would not
+//     fit, separate rings of three weight and two x buffers, 160 KiB: 94 instead of 102 us for Qwen3-8B
 //     at 256 tokens, the same at 8192): rows of 128
 //     bytes (one 64-k line per row), so each direct-to-LDS load (global_load_lds_dwordx4)
 //     moves 8 rows x 128 B; 16-byte chunks XOR-swizzled by row & 7 so the fragment reads
@@ -35,8 +35,9 @@
 //
 // Measured on MI355X (bf16, µs; this kernel at the better column tile / hipBLASLt +
 // silu_and_mul): Qwen3-8B 256 tokens 70.0 / 72.6, 8192 tokens 1286 / 1235; Qwen2.5-7B 256
-// tokens 110 / 88.5, 8192 tokens 1791 / 1834. The library therefore keeps the unfused pair
-// by default at these sizes and runs this kernel when the fused form is asked for.
+// tokens 110 / 88.5, 8192 tokens 1791 / 1834. Over an unpacked weight the library therefore
+// keeps the unfused pair by default at these sizes and runs this kernel when the fused form is
+// asked for. Packed weights have a kernel of their own (k_gate_up_silu_gemm_frag, below).
 #include <algorithm>
 #include <type_traits>
 
@@ -419,7 +420,8 @@ k_gate_up_silu_gemm(GemmArgs a) {
 //     of 128 bytes, 16-byte chunks XOR-swizzled by row & 7). The buffer form matters: after a
 //     global_load_lds the compiler treats every wait as one for a flat access and drains both
 //     counters (vmcnt(0) lgkmcnt(0)), after a buffer load it counts;
-//   * x fragments: a register ring of four (six in 192-token tiles), each refilled behind the MFMAs that used it last;
+//   * x fragments: a register ring of four (six in 192-token, two in 64-token tiles), each
+//     refilled behind the MFMAs that used it last;
 //   * one barrier per stage, in its middle, where the next step's operands are already in
 //     registers: no read waits for it.
 // The k order of every accumulator and the epilogue are k_gate_up_silu_gemm's, so the results

@@ -16,11 +16,10 @@ silu_and_mul) on MI355X: Qwen3-8B (H 4096, I 12288) 40 vs 45 us at 1-16 tokens, 
 (H 3584, I 18944) 54.5 vs 54.8 us. From 32 tokens on the library GEMM was as fast or faster,
 so the unfused pair runs there; `fused=True` forces the kernel (up to 64 tokens; above, the
 prefill-size MFMA GEMM with the activation as its epilogue, `gate_up_silu_gemm`, which also
-never materialises the [T, 2I] projection) and `fused=False` the pair. Over a weight packed at load time (`packed=`) the kernel runs by
-default up to PACKED_FUSED_TOKENS: 35.3 vs 46.1 us at 16 tokens and 37.1 vs 45.8 at 32
-(Qwen3-8B), 52.0 vs 56.7 at 32 (Qwen2.5-7B); at 48-64 tokens it is ahead at Qwen3-8B
-(44.5 vs 47.8) and behind at Qwen2.5-7B (65.0 vs 63.0). Above that the packed GEMM runs by
-default where `packed_gemm_default` says so, else the pair. Where no kernel applies (fp32,
+never materialises the [T, 2I] projection) and `fused=False` the pair. Over a weight packed
+at load time (`packed=`) the kernel runs by default up to PACKED_FUSED_TOKENS: 35.3 vs 46.1
+us at 16 tokens and 37.1 vs 45.8 at 32 (Qwen3-8B), 52.0 vs 56.7 at 32 (Qwen2.5-7B). Above
+that the packed GEMM runs by default where `packed_gemm_default` says so, else the pair. Where no kernel applies (fp32,
 shapes that are not multiples of 64, unaligned operands) the pair runs. CPU tensors, or
 `EMBERSERVE_FUSED_OPS=0`, take the eager forms.
 
