@@ -131,7 +131,8 @@ struct MlaArgs {
   float* part_o;               // [..][nh][dl]
   uint32_t* counters;          // [nseq][nh] split arrivals (MFMA kernel), zero between launches
   int32_t merge_apart;         // MFMA kernels: publish the partials only, k_mla_merge merges
-  int32_t balance;             // MFMA kernels: split sizes from all contexts (nseq <= 64), see mla_plan
+  int32_t balance;             // register MFMA kernel: split sizes from all contexts (nseq <= 64), see mla_plan;
+                               // the kernels' BAL (as a branch the plan's code cost other grids 0.3 us)
   uint32_t* err;
 };
 
@@ -222,10 +223,11 @@ struct SplitPlan {
 struct MlaPlan {
   int raw, per, n, first;  // balance: lane b's sequence (raw: its context length as given)
 };
+template <bool BAL>
 __device__ __forceinline__ MlaPlan mla_plan(const MlaArgs& a) {
   const int lane = threadIdx.x & (kWave - 1);
   MlaPlan p{0, 0, 0, 0};
-  if (!a.balance) return p;
+  if (!BAL) return p;
   const bool in = lane < a.nseq;
   p.raw = in ? a.ctx[lane] : 0;
   const int nt = (min(max(p.raw, 0), a.max_blocks * a.block_size) + kTile - 1) / kTile;
@@ -241,8 +243,9 @@ __device__ __forceinline__ MlaPlan mla_plan(const MlaArgs& a) {
   return p;
 }
 // Sequence b's part of the plan (b uniform); c: its context length as given.
+template <bool BAL>
 __device__ __forceinline__ SplitPlan seq_plan(const MlaArgs& a, const MlaPlan& p, int b, int& c) {
-  if (a.balance) {
+  if (BAL) {
     c = __builtin_amdgcn_readlane(p.raw, b);
     return {__builtin_amdgcn_readlane(p.first, b), p.per, __builtin_amdgcn_readlane(p.n, b)};
   }
@@ -257,6 +260,7 @@ __device__ __forceinline__ SplitPlan seq_plan(const MlaArgs& a, const MlaPlan& p
 // its XCD, whose L2 then holds their common rows. The units of a group of eight are rotated
 // by the group's number, so that no XCD gets one split number (or every eighth sequence)
 // alone.
+template <bool BAL>
 __device__ __forceinline__ void mla_unit(const MlaArgs& a, const MlaPlan& p, int& b, int& split, int& hc) {
   const int pid = blockIdx.x + gridDim.x * blockIdx.y;
   const int units8 = (a.nseq * a.splits) & ~7;
@@ -272,9 +276,9 @@ __device__ __forceinline__ void mla_unit(const MlaArgs& a, const MlaPlan& p, int
     u = units8 + r % rem;
     hc = r / rem;
   }
-  u = __builtin_amdgcn_readfirstlane(u);
-  if (a.balance) {  // the last sequence whose units begin at or before u (they begin in order)
+  if (BAL) {  // the last sequence whose units begin at or before u (they begin in order)
     const int lane = threadIdx.x & (kWave - 1);
+    u = __builtin_amdgcn_readfirstlane(u);
     b = __builtin_popcountll(__ballot(lane < a.nseq && p.first <= u)) - 1;
     split = u - __builtin_amdgcn_readlane(p.first, b);
   } else {
@@ -457,7 +461,7 @@ __device__ __forceinline__ void poison_state(float& m, float& lsum, f32x4 (&o)[N
   for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x4{m, m, m, m};
 }
 
-template <typename T, int DL, int DR, int NP, bool PSYNC, bool NT>
+template <typename T, int DL, int DR, int NP, bool PSYNC, bool NT, bool BAL>
 __global__ void __launch_bounds__(NP * 2 * kWave, 2)
 k_mla_mfma(MlaArgs a) {
   using M = MlaMfma<T>;
@@ -487,14 +491,14 @@ k_mla_mfma(MlaArgs a) {
   const int n = lane & 15;
   const int g = lane >> 4;
 
-  const MlaPlan all = mla_plan(a);
+  const MlaPlan all = mla_plan<BAL>(a);
   int b, split, hc;
-  mla_unit(a, all, b, split, hc);
+  mla_unit<BAL>(a, all, b, split, hc);
   const int head0 = hc * 16;
   const int nhc = min(16, a.nh - head0);
 
   int raw;
-  const SplitPlan plan = seq_plan(a, all, b, raw);
+  const SplitPlan plan = seq_plan<BAL>(a, all, b, raw);
   const int ctx = seq_context(a, raw);
   if (split >= plan.n) return;
   const int t0 = split * plan.per;
@@ -772,14 +776,14 @@ k_mla_lds(MlaArgs a) {
   const int n = lane & 15;
   const int g = lane >> 4;
 
-  const MlaPlan all = mla_plan(a);
+  const MlaPlan all = mla_plan<false>(a);
   int b, split, hc;
-  mla_unit(a, all, b, split, hc);
+  mla_unit<false>(a, all, b, split, hc);
   const int head0 = hc * 16;
   const int nhc = min(16, a.nh - head0);
 
   int raw;
-  const SplitPlan plan = seq_plan(a, all, b, raw);
+  const SplitPlan plan = seq_plan<false>(a, all, b, raw);
   const int ctx = seq_context(a, raw);
   if (split >= plan.n) return;
   const int t0 = split * plan.per;
@@ -1124,7 +1128,7 @@ k_mla_reduce(MlaArgs a) {
 // a (sequence, head) row, all of whose splits' partials it merges online, eight splits'
 // loads in flight at a time. One 64-lane workgroup per 256 output floats spreads a lone
 // sequence's partials (16 heads x 512 floats per split) over 32 CUs.
-template <typename TO, int DL>
+template <typename TO, int DL, bool BAL>
 __global__ void __launch_bounds__(kWave)
 k_mla_merge(MlaArgs a) {
   constexpr int TPR = DL / 4;
@@ -1136,7 +1140,7 @@ k_mla_merge(MlaArgs a) {
   const int d = (t % TPR) * 4;
   const int b = row / a.nh;
   int raw;
-  const SplitPlan plan = seq_plan(a, mla_plan(a), b, raw);
+  const SplitPlan plan = seq_plan<BAL>(a, mla_plan<BAL>(a), b, raw);
   const int nsplit = plan.n;
   if (nsplit == 1) return;  // its only split wrote the output rows
   const int64_t stride = a.nh;
@@ -1182,12 +1186,27 @@ k_mla_merge(MlaArgs a) {
   store_pack<TO, 4>(static_cast<TO*>(a.out) + b * a.o_sb + h * a.o_sh + d, r);
 }
 
-template <typename T, bool NT>
+template <typename T>
+void launch_merge(const MlaArgs& a, uint32_t blocks, hipStream_t st) {
+  if (a.balance)
+    k_mla_merge<T, kMlaDL, true><<<blocks, kWave, 0, st>>>(a);
+  else
+    k_mla_merge<T, kMlaDL, false><<<blocks, kWave, 0, st>>>(a);
+}
+template <typename T, bool NT, bool BAL>
 void launch_register_mfma(const MlaArgs& a, dim3 grid, bool four, hipStream_t st) {
   if (four)
-    k_mla_mfma<T, kMlaDL, kMlaDR, kMlaPairsSmall, kMlaPairSync, NT><<<grid, kMlaPairsSmall * 2 * kWave, 0, st>>>(a);
+    k_mla_mfma<T, kMlaDL, kMlaDR, kMlaPairsSmall, kMlaPairSync, NT, BAL>
+        <<<grid, kMlaPairsSmall * 2 * kWave, 0, st>>>(a);
   else
-    k_mla_mfma<T, kMlaDL, kMlaDR, kMlaPairs, kMlaPairSync, NT><<<grid, kMlaPairs * 2 * kWave, 0, st>>>(a);
+    k_mla_mfma<T, kMlaDL, kMlaDR, kMlaPairs, kMlaPairSync, NT, BAL><<<grid, kMlaPairs * 2 * kWave, 0, st>>>(a);
+}
+template <typename T, bool NT>
+void launch_register_mfma(const MlaArgs& a, dim3 grid, bool four, hipStream_t st) {
+  if (a.balance)
+    launch_register_mfma<T, NT, true>(a, grid, four, st);
+  else
+    launch_register_mfma<T, NT, false>(a, grid, four, st);
 }
 
 template <typename T>
@@ -1326,7 +1345,7 @@ int ember_mla_decode(const void* q_c, int64_t qc_seq_stride, int64_t qc_head_str
     // 34.8, 48 x 4096 36.0 -> 29.8, 64 x 8192 71.1 -> 58.1, 16 x 8192 29.0 -> 27.8; contexts of one
     // length pay the plan, 32 x 4096 34.0 -> 34.3, 16 x 8192 33.8 -> 34.7. Below: 16 x 4096 20.4 -> 22.1.
     // (The other bounds: one lane per sequence, and the sums of mla_plan's divisions.)
-    a.balance = a.merge_apart && num_seqs > 1 && num_seqs <= kWave && max_blocks * block_size >= num_splits * 512 &&
+    a.balance = !small && a.merge_apart && num_seqs > 1 && num_seqs <= kWave && max_blocks * block_size >= num_splits * 512 &&
                 num_seqs * (max_blocks * block_size / kTile + 1 + num_splits) <= (1 << 20);
     if (q_dtype == EMBER_F16)
       launch_mfma<_Float16>(a, grid, small, four, st);
@@ -1336,9 +1355,9 @@ int ember_mla_decode(const void* q_c, int64_t qc_seq_stride, int64_t qc_head_str
       const int64_t threads = num_seqs * num_heads * (kMlaDL / 4);
       const uint32_t blocks = static_cast<uint32_t>((threads + kWave - 1) / kWave);
       if (q_dtype == EMBER_F16)
-        k_mla_merge<_Float16, kMlaDL><<<blocks, kWave, 0, st>>>(a);
+        launch_merge<_Float16>(a, blocks, st);
       else
-        k_mla_merge<__bf16, kMlaDL><<<blocks, kWave, 0, st>>>(a);
+        launch_merge<__bf16>(a, blocks, st);
     }
   } else {
     dim3 grid(static_cast<uint32_t>(num_seqs * num_heads), static_cast<uint32_t>(num_splits));
