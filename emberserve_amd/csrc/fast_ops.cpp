@@ -7,8 +7,8 @@
 // eager form. Ordinary means: plain CUDA tensors of one device, which is the current one
 // (no subclass, no functorch or dispatch-mode wrapper, no tracing), the dtypes and strides
 // the kernels read as they are, EMBERSERVE_FUSED_OPS not "0", EMBERSERVE_CHECK_INDICES not
-// "1", and an entry point that accepted the call. No state is kept but the entry points'
-// addresses (set once per loaded library).
+// "1", and an entry point that accepted the call. A launch that fails is raised. No state is
+// kept but the entry points' addresses (set once per loaded library).
 //
 // What bounded the small calls was this host work: about 16 us a launch in Python and ctypes,
 // 5 here, 3-4 of them the launch itself. Measured (wall per pass, launches back to back): the
@@ -31,6 +31,8 @@
 #include <cstdlib>
 #include <cstring>
 #include <initializer_list>
+#include <stdexcept>
+#include <string>
 
 #include "../../include/ember_ops.h"
 
@@ -43,13 +45,13 @@ struct Entry {
 };
 enum {
   kRmsnorm, kAddRmsnorm, kRope, kSilu, kEmbedding, kQkNormRope, kMlaLatentRope, kRopeKvCache, kMlaLatentRopeCache,
-  kPagedDecode, kMlaDecode, kEntries
+  kPagedDecode, kMlaDecode, kStatusString, kEntries
 };
 Entry g_entry[kEntries] = {
     {"ember_rmsnorm", nullptr}, {"ember_fused_add_rmsnorm", nullptr}, {"ember_rope", nullptr},
     {"ember_silu_and_mul", nullptr}, {"ember_embedding", nullptr}, {"ember_qk_norm_rope", nullptr},
     {"ember_mla_latent_rope", nullptr}, {"ember_rope_kv_cache", nullptr}, {"ember_mla_latent_rope_cache", nullptr},
-    {"ember_paged_decode", nullptr}, {"ember_mla_decode", nullptr}};
+    {"ember_paged_decode", nullptr}, {"ember_mla_decode", nullptr}, {"ember_status_string", nullptr}};
 bool g_bound = false;
 
 #define ENTRY(i, f) reinterpret_cast<decltype(&f)>(g_entry[i].fn)
@@ -167,6 +169,17 @@ int launch(F&& f) {
   return st;
 }
 
+// Whether entry point `e` answered the call: false for a refusal, which comes before any launch.
+// A failed launch is raised, as the wrappers raise it: the kernel may have been enqueued (the
+// status is the thread's last HIP error, which can be an earlier call's), and a second run
+// would rotate in-place operands twice.
+bool answered(int st, int e) {
+  if (st == EMBER_OK) return true;
+  if (st == EMBER_EINVAL || st == EMBER_EALIGN || st == EMBER_ENODEV || st == EMBER_ETOOBIG) return false;
+  throw std::runtime_error(std::string("emberserve_amd: ") + g_entry[e].name + " failed: " +
+                           ENTRY(kStatusString, ember_status_string)(st) + " (status " + std::to_string(st) + ")");
+}
+
 PyObject* pair(PyObject* a, PyObject* b) {  // steals both
   PyObject* t = a != nullptr && b != nullptr ? PyTuple_New(2) : nullptr;
   if (t == nullptr) {
@@ -212,7 +225,7 @@ PyObject* rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return ENTRY(kRmsnorm, ember_rmsnorm)(x->data_ptr(), r.stride, w->data_ptr(), dtype_tag(*w), out.data_ptr(),
                                           r.width, r.rows, r.width, static_cast<float>(eps), tag, s);
   });
-  if (st != EMBER_OK) Py_RETURN_NONE;
+  if (!answered(st, kRmsnorm)) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
@@ -241,7 +254,7 @@ PyObject* add_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                                        sum.data_ptr(), r.width, r.rows, r.width,
                                                        static_cast<float>(eps), tag, s);
   });
-  if (st != EMBER_OK) Py_RETURN_NONE;
+  if (!answered(st, kAddRmsnorm)) Py_RETURN_NONE;
   return pair(THPVariable_Wrap(std::move(out)), THPVariable_Wrap(std::move(sum)));
   END_HANDLE_TH_ERRORS
 }
@@ -263,7 +276,7 @@ PyObject* silu_and_mul(PyObject*, PyObject* arg) {
   const int st = launch([&] {
     return ENTRY(kSilu, ember_silu_and_mul)(x->data_ptr(), r.stride, out.data_ptr(), inter, r.rows, inter, tag, s);
   });
-  if (st != EMBER_OK) Py_RETURN_NONE;
+  if (!answered(st, kSilu)) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
@@ -288,7 +301,7 @@ PyObject* embedding(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                               w->data_ptr(), w->size(0), w->size(1), w->stride(0), out.data_ptr(),
                                               w->size(1), static_cast<int64_t>(w->element_size()), s);
   });
-  if (st != EMBER_OK) Py_RETURN_NONE;
+  if (!answered(st, kEmbedding)) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
@@ -317,7 +330,7 @@ PyObject* rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                     static_cast<const float*>(sin->data_ptr()), cos->size(0), cos->stride(0),
                                     static_cast<const int64_t*>(pos->data_ptr()), q->size(0), tag, s);
   });
-  if (st != EMBER_OK) Py_RETURN_NONE;
+  if (!answered(st, kRope)) Py_RETURN_NONE;
   return pair(Py_NewRef(a[0]), Py_NewRef(a[1]));
   END_HANDLE_TH_ERRORS
 }
@@ -344,7 +357,7 @@ PyObject* qk_norm_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
         static_cast<const float*>(cos->data_ptr()), static_cast<const float*>(sin->data_ptr()), cos->size(0),
         cos->stride(0), static_cast<const int64_t*>(pos->data_ptr()), q->size(0), tag, s);
   });
-  if (st != EMBER_OK) Py_RETURN_NONE;
+  if (!answered(st, kQkNormRope)) Py_RETURN_NONE;
   return pair(Py_NewRef(a[0]), Py_NewRef(a[1]));
   END_HANDLE_TH_ERRORS
 }
@@ -385,7 +398,7 @@ PyObject* rope_kv_cache(PyObject*, PyObject* const* a, Py_ssize_t n) {
         static_cast<const int64_t*>(pos->data_ptr()), static_cast<const int64_t*>(slots->data_ptr()), t,
         kc->data_ptr(), vc->data_ptr(), nslots, slot_stride, kc->stride(2), tag, s);
   });
-  if (st != EMBER_OK) Py_RETURN_NONE;
+  if (!answered(st, kRopeKvCache)) Py_RETURN_NONE;
   return pair(Py_NewRef(a[0]), Py_NewRef(a[1]));
   END_HANDLE_TH_ERRORS
 }
@@ -419,7 +432,7 @@ PyObject* mla_latent_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
         static_cast<const float*>(cos->data_ptr()), static_cast<const float*>(sin->data_ptr()), cos->size(0),
         cos->stride(0), static_cast<const int64_t*>(pos->data_ptr()), t, latent.data_ptr(), r + dr, tag, s);
   });
-  if (st != EMBER_OK) Py_RETURN_NONE;
+  if (!answered(st, kMlaLatentRope)) Py_RETURN_NONE;
   return pair(Py_NewRef(a[2]), THPVariable_Wrap(std::move(latent)));
   END_HANDLE_TH_ERRORS
 }
@@ -455,7 +468,7 @@ PyObject* mla_latent_rope_cache(PyObject*, PyObject* const* a, Py_ssize_t n) {
         keep ? r + dr : 0, static_cast<const int64_t*>(slots->data_ptr()), cache->data_ptr(), nslots, slot_stride, tag,
         s);
   });
-  if (st != EMBER_OK) Py_RETURN_NONE;
+  if (!answered(st, kMlaLatentRopeCache)) Py_RETURN_NONE;
   return pair(Py_NewRef(a[2]), keep ? THPVariable_Wrap(std::move(latent)) : Py_NewRef(Py_None));
   END_HANDLE_TH_ERRORS
 }
@@ -524,7 +537,7 @@ PyObject* paged_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
         static_cast<const int32_t*>(ctx->data_ptr()), b, h, static_cast<float>(scale), p.splits, 0, p.ws, p.ws_bytes,
         out.data_ptr(), out.stride(0), out.stride(1), s);
   });
-  if (st != EMBER_OK) Py_RETURN_NONE;
+  if (!answered(st, kPagedDecode)) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
@@ -559,7 +572,7 @@ PyObject* mla_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
         static_cast<const int32_t*>(ctx->data_ptr()), b, h, static_cast<float>(scale), p.splits, p.ws, p.ws_bytes,
         out.data_ptr(), out.stride(0), out.stride(1), s);
   });
-  if (st != EMBER_OK) Py_RETURN_NONE;
+  if (!answered(st, kMlaDecode)) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }

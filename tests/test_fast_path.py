@@ -5,6 +5,7 @@ the others (which the wrappers convert, refuse or run eagerly)."""
 
 from __future__ import annotations
 
+import ctypes
 import subprocess
 import sys
 
@@ -203,6 +204,40 @@ def test_other_calls_are_left_to_the_python_wrappers(monkeypatch):
     assert seen == [None]
     with pytest.raises(ValueError):
         ops.rmsnorm(x, w[:32], 1e-6)
+
+
+@gpu
+def test_a_failed_launch_is_raised_and_not_run_again(monkeypatch):
+    """EMBER_ELAUNCH can come with the kernel enqueued (an earlier, uncleared HIP error), so no
+    wrapper may run the call a second time: in place, that would rotate q and k twice. The
+    status is forced by stub entry points; nothing is launched."""
+    from emberserve_amd import _fast
+    lib, st = _lib.load(), 3
+    real = {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _lib.SIGNATURES}
+    names = ("ember_rope", "ember_rope_kv_cache", "ember_rmsnorm", "ember_paged_decode")
+    stubs = [ctypes.CFUNCTYPE(ctypes.c_int, *_lib.SIGNATURES[n])(lambda *a: st) for n in names]
+    again = []
+    for name in ("rope_hip", "rope_kv_cache_hip", "rmsnorm_hip"):
+        monkeypatch.setattr(ops, name, lambda *a, name=name: again.append(name))
+    q, k, v = _rand(3, 4, 64), _rand(3, 2, 64, seed=1), _rand(3, 2, 64, seed=2)
+    cos, sin = RotaryEmbedding(64, 16, 1e4).full_tables(q.device)
+    pos = torch.arange(3, device=DEV)
+    caches = [torch.zeros(1, 16, 2, 64, dtype=q.dtype, device=DEV) for _ in range(2)]
+    dec = [t.to(DEV) for t in gen.decode_inputs([5, 7], 4, 2, 64, 16, torch.bfloat16, seed=1)]
+    calls = {"rope": lambda: ops.rope(q, k, cos, sin, pos),
+             "rope_kv_cache": lambda: ops.rope_kv_cache(q, k, v, cos, sin, pos, pos, *caches),
+             "rmsnorm": lambda: ops.rmsnorm(q.view(3, -1), _rand(256), 1e-6),
+             "paged_decode": lambda: paged_attention_decode(*dec, 0.1)}
+    _fast.bind({**real, **{n: ctypes.cast(s, ctypes.c_void_p).value for n, s in zip(names, stubs)}})
+    try:
+        for what, call in calls.items():
+            with pytest.raises(RuntimeError, match=f"ember_{what} failed.*status 3"):
+                call()
+        st = 1  # refused before any launch: the wrappers' turn
+        calls["rope"]()
+        assert again == ["rope_hip"]
+    finally:
+        _fast.bind(real)
 
 
 @gpu
