@@ -249,15 +249,17 @@ def gate_up_silu(x: Tensor, weight: Tensor | None, *, num_workgroups: int | None
     """silu_and_mul(F.linear(x, weight)) with weight [2I, H] (qwen2.py:60-61). With `packed`
     (`pack_gate_up_weight(weight)`), the fused kernel reads the packed copy instead. With
     `packed` and weight None (a model that dropped the unpacked weight) every size runs on
-    the packed copy: the decode kernel up to PACKED_FUSED_TOKENS tokens, the packed prefill
-    GEMM above (33-64 tokens, us, decode kernel | GEMM: Qwen3-8B 39-42 | 40-41, Qwen2.5-7B 63-68
-    | 50, Qwen2.5-0.5B 12 | 9)."""
+    the packed copy: the decode kernel up to PACKED_FUSED_TOKENS tokens (PACKED_MAX_TOKENS when
+    num_workgroups, which is the decode kernel's, is given), the packed prefill GEMM above
+    (33-64 tokens, us, decode kernel | GEMM: Qwen3-8B 39-42 | 40-41, Qwen2.5-7B 63-68 | 50,
+    Qwen2.5-0.5B 12 | 9)."""
     if weight is None:
         if packed is None:
             raise ValueError("gate_up_silu: weight None needs the packed weight")
         if fused is False:
             raise ValueError("gate_up_silu: the unfused pair needs the unpacked weight")
-        if x.reshape(-1, packed.hidden).shape[0] > PACKED_FUSED_TOKENS:
+        limit = PACKED_FUSED_TOKENS if num_workgroups is None else PACKED_MAX_TOKENS
+        if x.reshape(-1, packed.hidden).shape[0] > limit:
             return gate_up_silu_gemm_packed(x, packed)
         return _packed_decode(x, packed, num_workgroups)
     return _gate_up_silu_decode(x, weight, num_workgroups, fused, packed)

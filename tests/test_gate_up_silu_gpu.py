@@ -393,3 +393,15 @@ def test_fused_true_past_64_tokens_runs_the_gemm():
     w48 = (torch.randn(2 * 48, 512, generator=g) / 512 ** 0.5).to(torch.bfloat16).to(DEV)
     x = (torch.randn(100, 512, generator=g) * 0.5).to(torch.bfloat16).to(DEV)
     assert torch.equal(gate_up_silu(x, w48, fused=True), gate_up_silu_torch(x, w48))
+
+@pytest.mark.parametrize("tokens", [16, 48, 64])
+def test_packed_only_keeps_the_given_workgroups(tokens):
+    """With the packed copy alone, num_workgroups means the decode kernel up to its 64 tokens:
+    the packing's own count gives its bits, another one is refused."""
+    from emberserve_amd.gate_up_silu import pack_gate_up_weight
+    x, w = gen.gate_up_inputs(tokens, 256, 256, torch.bfloat16, seed=31)
+    dx, packed = x.to(DEV), pack_gate_up_weight(w.to(DEV), num_workgroups=7)
+    _say(f"packed only T={tokens} num_workgroups")
+    _check(gate_up_silu(dx, None, packed=packed, num_workgroups=7), x, w, f"T={tokens}")
+    with pytest.raises(ValueError, match="packed for 7 workgroups"):
+        gate_up_silu(dx, None, packed=packed, num_workgroups=8)
