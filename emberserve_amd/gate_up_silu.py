@@ -320,7 +320,7 @@ def _gate_up_silu_decode(x: Tensor, weight: Tensor, num_workgroups: int | None, 
         # the fused form asked for at prefill sizes: the MFMA GEMM with the activation epilogue
         return gate_up_silu_gemm(x, weight, column_tile=gemm_column_tile(T, I, x.device))
     if (fused is None and T > default and packed is not None and num_workgroups is None
-            and _gemm_fits(x2, weight, out) and packed_gemm_default(T, H, I, x.device)
+            and _gemm_fits(x2, weight, out) and x2.stride(0) >= H and packed_gemm_default(T, H, I, x.device)
             and (packed.hidden, packed.inter, packed.dtype, packed.device) == (H, I, x.dtype, x.device)):
         _launch_gemm_packed(x2, packed, out)
         return out.view(*x.shape[:-1], I)

@@ -405,3 +405,15 @@ def test_packed_only_keeps_the_given_workgroups(tokens):
     _check(gate_up_silu(dx, None, packed=packed, num_workgroups=7), x, w, f"T={tokens}")
     with pytest.raises(ValueError, match="packed for 7 workgroups"):
         gate_up_silu(dx, None, packed=packed, num_workgroups=8)
+
+
+def test_overlapping_rows_run_the_pair():
+    """x rows closer together than H (one row expanded, sliding windows) are no operand of the
+    packed GEMM: the unfused pair runs, as without the packed copy."""
+    from emberserve_amd.gate_up_silu import pack_gate_up_weight
+    x, w = gen.gate_up_inputs(2, 256, 256, torch.bfloat16, seed=32)
+    dx, dw = x.to(DEV), w.to(DEV)
+    packed = pack_gate_up_weight(dw)
+    for view in (dx[:1].expand(48, 256), dx.view(-1).as_strided((32 + 1, 256), (8, 1))):
+        _say(f"overlapping rows, strides {tuple(view.stride())}")
+        assert torch.equal(gate_up_silu(view, dw, packed=packed), gate_up_silu_torch(view, dw))
