@@ -11,6 +11,7 @@ import threading
 from pathlib import Path
 
 import torch
+from torch.compiler import is_dynamo_compiling as tracing  # noqa: F401  (for the callers of `fast`)
 
 LIB_PATH = Path(__file__).resolve().parent / "libember_ops.so"
 ABI_VERSION = 18

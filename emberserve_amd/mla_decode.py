@@ -114,7 +114,7 @@ def mla_decode(q_abs: Tensor | tuple[Tensor, Tensor], latent_cache: Tensor, bloc
     else:
         q_c, q_pe = q_abs[..., :DL], q_abs[..., DL:]
         D = q_abs.shape[2]
-    if num_splits is None and out is None and q_c.dim() == 3 and q_c.shape[2] == DL:
+    if num_splits is None and out is None and q_c.dim() == 3 and q_c.shape[2] == DL and not _lib.tracing():
         got = _lib.fast.mla_decode(q_c, q_pe, latent_cache, block_tables, context_lens, scale, _plan)
         if got is not None:  # an ordinary call, answered by the native host path
             return got

@@ -31,7 +31,7 @@ import os
 import torch
 
 from . import _lib
-from ._lib import fast
+from ._lib import fast, tracing
 from .eager import (  # noqa: F401  (re-exported: the reference's names)
     _rotate_half,
     embedding_torch,
@@ -502,10 +502,11 @@ def mla_latent_rope_cache_hip(c: torch.Tensor, k_pe: torch.Tensor, q_pe: torch.T
 #
 # An ordinary GPU call is answered by the native host path (`fast`, csrc/fast_ops.cpp), which
 # returns None, with nothing launched, for every other one: CPU tensors, the opt-out, index
-# checks, operands that need a conversion, and whatever is to be refused.
+# checks, operands that need a conversion, and whatever is to be refused. While torch.compile
+# traces it is not called: Dynamo cannot enter a C function (`tracing` costs 0.04 us).
 
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
-    got = fast.rmsnorm(x, weight, eps)
+    got = None if tracing() else fast.rmsnorm(x, weight, eps)
     if got is not None:
         return got
     if fused_enabled(x):
@@ -515,7 +516,7 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
 
 def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
                       eps: float) -> tuple[torch.Tensor, torch.Tensor]:
-    got = fast.add_rmsnorm(x, residual, weight, eps)
+    got = None if tracing() else fast.add_rmsnorm(x, residual, weight, eps)
     if got is not None:
         return got
     if fused_enabled(x):
@@ -525,7 +526,7 @@ def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Ten
 
 def rope(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
          positions: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
-    got = fast.rope(q, k, cos, sin, positions)
+    got = None if tracing() else fast.rope(q, k, cos, sin, positions)
     if got is not None:
         return got
     if fused_enabled(q):
@@ -534,7 +535,7 @@ def rope(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
 
 
 def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
-    got = fast.silu_and_mul(x)
+    got = None if tracing() else fast.silu_and_mul(x)
     if got is not None:
         return got
     if fused_enabled(x):
@@ -543,7 +544,7 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
 
 
 def embedding(ids: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    got = fast.embedding(ids, weight)
+    got = None if tracing() else fast.embedding(ids, weight)
     if got is not None:
         return got
     if fused_enabled(weight):
@@ -554,7 +555,7 @@ def embedding(ids: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 def qk_norm_rope(q: torch.Tensor, k: torch.Tensor, q_weight: torch.Tensor, k_weight: torch.Tensor,
                  eps: float, cos: torch.Tensor, sin: torch.Tensor,
                  positions: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
-    got = fast.qk_norm_rope(q, k, q_weight, k_weight, eps, cos, sin, positions)
+    got = None if tracing() else fast.qk_norm_rope(q, k, q_weight, k_weight, eps, cos, sin, positions)
     if got is not None:
         return got
     if fused_enabled(q):
@@ -565,7 +566,7 @@ def qk_norm_rope(q: torch.Tensor, k: torch.Tensor, q_weight: torch.Tensor, k_wei
 def mla_latent_rope(c: torch.Tensor, k_pe: torch.Tensor, q_pe: torch.Tensor, weight: torch.Tensor,
                     eps: float, cos: torch.Tensor, sin: torch.Tensor,
                     positions: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
-    got = fast.mla_latent_rope(c, k_pe, q_pe, weight, eps, cos, sin, positions)
+    got = None if tracing() else fast.mla_latent_rope(c, k_pe, q_pe, weight, eps, cos, sin, positions)
     if got is not None:
         return got
     if fused_enabled(c):
@@ -590,8 +591,8 @@ def rope_kv_cache(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.
                   positions: torch.Tensor, slot_mapping: torch.Tensor, k_cache: torch.Tensor,
                   v_cache: torch.Tensor, q_weight: torch.Tensor | None = None,
                   k_weight: torch.Tensor | None = None, eps: float = 1e-6) -> tuple[torch.Tensor, torch.Tensor]:
-    got = fast.rope_kv_cache(q, k, v, cos, sin, positions, slot_mapping, k_cache, v_cache, q_weight, k_weight,
-                             eps)
+    got = None if tracing() else fast.rope_kv_cache(q, k, v, cos, sin, positions, slot_mapping, k_cache, v_cache,
+                                                    q_weight, k_weight, eps)
     if got is not None:
         return got
     if fused_enabled(q):
@@ -609,8 +610,8 @@ def mla_latent_rope_cache(c: torch.Tensor, k_pe: torch.Tensor, q_pe: torch.Tenso
                           eps: float, cos: torch.Tensor, sin: torch.Tensor, positions: torch.Tensor,
                           slot_mapping: torch.Tensor, cache: torch.Tensor,
                           return_latent: bool = True) -> tuple[torch.Tensor, torch.Tensor | None]:
-    got = fast.mla_latent_rope_cache(c, k_pe, q_pe, weight, eps, cos, sin, positions, slot_mapping, cache,
-                                     return_latent)
+    got = None if tracing() else fast.mla_latent_rope_cache(c, k_pe, q_pe, weight, eps, cos, sin, positions,
+                                                            slot_mapping, cache, return_latent)
     if got is not None:
         return got
     if fused_enabled(c):

@@ -169,7 +169,7 @@ def paged_attention_decode(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_ta
     """One-token-per-sequence paged attention (paged_triton.py:323-399). `num_warps` is
     accepted for signature compatibility; the kernel's workgroup shape is fixed."""
     del num_warps
-    if num_splits is None and out is None and variant is None:
+    if num_splits is None and out is None and variant is None and not _lib.tracing():
         got = _lib.fast.paged_decode(q, k_cache, v_cache, block_tables, context_lens, scale, _plan)
         if got is not None:  # an ordinary call, answered by the native host path
             return got
