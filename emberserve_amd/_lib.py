@@ -14,7 +14,7 @@ import torch
 from torch.compiler import is_dynamo_compiling as tracing  # noqa: F401  (for the callers of `fast`)
 
 LIB_PATH = Path(__file__).resolve().parent / "libember_ops.so"
-ABI_VERSION = 18
+ABI_VERSION = 19
 
 F32, F16, BF16 = 0, 1, 2
 ERR_EMBED_ID = 1
@@ -106,6 +106,7 @@ SIGNATURES: dict[str, list] = {
     "ember_moe_align_workspace_bytes": [_i64, _i64],
     "ember_moe_align": [_p, _i32, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _p],
     "ember_read_errors": [ctypes.POINTER(ctypes.c_uint32), _i32],
+    "ember_stream_capture_id": [_p, ctypes.POINTER(ctypes.c_uint64)],
     "ember_abi_version": [],
     "ember_status_string": [_i32],
 }

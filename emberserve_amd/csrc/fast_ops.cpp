@@ -590,7 +590,7 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_fast", nullptr, -1, kMethods, nu
 PyMODINIT_FUNC PyInit__fast(void) {
   PyObject* m = PyModule_Create(&kModule);
   // the ABI version (ember_abi_version) of the header this was compiled against
-  if (m != nullptr && PyModule_AddIntConstant(m, "ABI_VERSION", 18) != 0) {
+  if (m != nullptr && PyModule_AddIntConstant(m, "ABI_VERSION", 19) != 0) {
     Py_DECREF(m);
     return nullptr;
   }

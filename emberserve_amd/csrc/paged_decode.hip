@@ -780,9 +780,9 @@ int64_t ember_paged_decode_workspace_bytes(int64_t num_seqs, int64_t num_heads, 
 namespace ember {
 namespace {
 
-// ember_paged_decode's body. `counters` (when non-null) replaces the arrival counters at the
-// end of the workspace: the no-allocation entry point keeps them at a fixed place, so that
-// calls of different shapes always find them at zero.
+// ember_paged_decode's body. The arrival counters are the workspace's last words, whatever part
+// of it the call's partials need, so that calls of different shapes on one buffer find them at
+// zero; `counters` (when non-null) replaces them (the no-allocation entry point's fixed place).
 int paged_decode_core(const void* q, int64_t q_seq_stride, int64_t q_head_stride, int q_dtype,
                       const void* k_cache, const void* v_cache, int64_t num_blocks, int64_t block_size,
                       int64_t num_kv_heads, int64_t head_dim, int64_t k_block_stride, int64_t k_slot_stride,
@@ -845,7 +845,11 @@ int paged_decode_core(const void* q, int64_t q_seq_stride, int64_t q_head_stride
     a.part_m = ws;
     a.part_l = ws + rows;
     a.part_o = ws + 2 * rows;
-    a.counters = counters != nullptr ? counters : reinterpret_cast<uint32_t*>(ws + rows * (head_dim + 2));
+    const int64_t counter_bytes = need - rows * (head_dim + 2) * int64_t(sizeof(float));
+    a.counters = counters != nullptr
+                     ? counters
+                     : reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) +
+                                                   ((workspace_bytes - counter_bytes) & ~int64_t(3)));
   }
   a.err = err;
   hipStream_t st = static_cast<hipStream_t>(stream);

@@ -45,7 +45,7 @@ __host__ int device_cu_count() {
 
 extern "C" {
 
-int ember_abi_version(void) { return 18; }
+int ember_abi_version(void) { return 19; }
 
 const char* ember_status_string(int status) {
   switch (status) {
@@ -70,6 +70,15 @@ int ember_read_errors(uint32_t* flags, int clear) {
     const uint32_t zero = 0;
     if (hipMemcpy(p, &zero, sizeof(zero), hipMemcpyHostToDevice) != hipSuccess) return EMBER_ENODEV;
   }
+  return EMBER_OK;
+}
+
+int ember_stream_capture_id(void* stream, uint64_t* id) {
+  if (id == nullptr) return EMBER_EINVAL;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long capture = 0;
+  if (hipStreamGetCaptureInfo(static_cast<hipStream_t>(stream), &status, &capture) != hipSuccess) return EMBER_ENODEV;
+  *id = status == hipStreamCaptureStatusActive ? capture : 0;
   return EMBER_OK;
 }
 

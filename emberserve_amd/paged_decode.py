@@ -13,8 +13,8 @@ in fp32 throughout. CPU tensors take the eager form of PagedTorchAttentionBacken
 (attn/paged_torch.py:87-98).
 
 The split count comes from shapes only (batch, table width), never from tensor values, so
-a captured HIP graph replays exactly what was captured; the split-K scratch is cached per
-shape for the same reason (paged_triton.py:293-310).
+a captured HIP graph replays exactly what was captured; the split-K scratch stays at the
+captured addresses for the same reason (paged_triton.py:293-310).
 """
 
 from __future__ import annotations
@@ -25,7 +25,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
-from ._scratch import ScratchCache, round_up
+from ._scratch import SharedScratch, round_up
 from .ops import _check_indices, _launch, _require_device
 
 BLOCK_MULTIPLE = 16
@@ -121,14 +121,17 @@ def default_variant() -> str:
     return v
 
 
-def _workspace_bytes(num_splits: int, batch: int, num_heads: int, head_dim: int) -> int:
-    return _lib.load().ember_paged_decode_workspace_bytes(batch, num_heads, head_dim, num_splits)
+# Split-K partials and arrival counters, one buffer per (thread, device, stream) for all shapes,
+# at addresses that stay valid for a graph replay (paged_triton.py:293-310); two streams never
+# share counters.
+_SCRATCH = SharedScratch("paged_attention_decode")
 
 
-# Split-K partials and arrival counters, cached per (num_splits, B, H, D, device, stream) so a
-# graph replay reads the addresses that were captured (paged_triton.py:293-310) and two
-# streams never share counters.
-_SCRATCH = ScratchCache("paged_attention_decode", min_bytes=16)
+def _workspace(num_splits: int, batch: int, num_heads: int, head_dim: int, device: torch.device) -> Tensor:
+    """The workspace of a call: ember_paged_decode_workspace_bytes of partials and, at the
+    buffer's end, counters."""
+    rows = batch * num_heads
+    return _SCRATCH.get(num_splits * rows * (head_dim + 2) * 4, round_up(rows * 4, 16), device)
 
 
 def _plan(B: int, H: int, D: int, Hkv: int, max_context: int, q: Tensor) -> tuple[int, Tensor | None]:
@@ -137,7 +140,7 @@ def _plan(B: int, H: int, D: int, Hkv: int, max_context: int, q: Tensor) -> tupl
     splits = max(1, min(splits, max(1, -(-max_context // TILE))))
     if splits == 1:
         return 1, None
-    return splits, _SCRATCH.get((splits, B, H, D), lambda: _workspace_bytes(splits, B, H, D), q.device)
+    return splits, _workspace(splits, B, H, D, q.device)
 
 
 def paged_decode_torch(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_tables: Tensor,
@@ -205,7 +208,7 @@ def paged_attention_decode(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_ta
     num_splits = max(1, min(int(num_splits), num_tiles_max))
     ws = None
     if num_splits > 1:
-        ws = _SCRATCH.get((num_splits, B, H, D), lambda: _workspace_bytes(num_splits, B, H, D), q.device)
+        ws = _workspace(num_splits, B, H, D, q.device)
     flags = _lib.DECODE_FP32 if variant == "sum" else 0
     _launch("ember_paged_decode", _lib.load().ember_paged_decode, q.device,
             q.data_ptr(), q.stride(0), q.stride(1), _lib.dtype_tag(q.dtype),
@@ -218,8 +221,8 @@ def paged_attention_decode(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_ta
             out.data_ptr(), out.stride(0), out.stride(1))
     if _check_indices():
         if ws is not None:
-            need = _workspace_bytes(num_splits, B, H, D)
-            _SCRATCH.verify_counters(ws, need - round_up(B * H * 4, 16), need - round_up(B * H * 4, 16) + B * H * 4)
+            start = ws.numel() * 4 - round_up(B * H * 4, 16)
+            _SCRATCH.verify_counters(ws, start, start + B * H * 4)
         flags = _lib.read_errors(clear=True)
         if flags & _lib.ERR_DECODE_CTX:
             raise IndexError("emberserve_amd.paged_attention_decode: context length outside the block table")

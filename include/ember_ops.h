@@ -110,6 +110,9 @@ const char* ember_status_string(int status);
  * zeroes it. Synchronises the device. Returns EMBER_OK or EMBER_ENODEV. */
 int ember_read_errors(uint32_t* flags, int clear);
 
+/* *id <- the id of the graph capture that `stream` takes part in, 0 when it is not capturing. */
+int ember_stream_capture_id(void* stream, uint64_t* id);
+
 /* RMSNorm of `rows` rows of `cols` elements:
  *   out = round(w * round(x * rsqrt(mean(x^2) + eps)))
  * fp32 math, rounding to `dtype` at the two points the reference rounds.
@@ -297,9 +300,12 @@ int64_t ember_paged_decode_workspace_bytes(int64_t num_seqs, int64_t num_heads, 
  * block_size must be a multiple of 16 and head_dim <= 256. With num_splits > 1 each
  * sequence's context is cut into num_splits key ranges whose partial results are merged by
  * the last split to finish (or a second kernel) through `workspace`
- * (ember_paged_decode_workspace_bytes bytes, 16-byte aligned, zero-filled before its first
- * use; every call leaves it ready for the next, and calls that overlap on one workspace
- * race); the split count changes rounding only, never which keys are seen.
+ * (at least ember_paged_decode_workspace_bytes bytes, 16-byte aligned, zero-filled before its
+ * first use; every call leaves it ready for the next, and calls that overlap on one workspace
+ * race). The partials are at its start and the counters are its last num_seqs x num_heads
+ * words (rounded up to 16 bytes), so calls of different shapes may take turns on one larger
+ * workspace of a fixed size as long as no call's partials reach another's counters; then only
+ * the counters have to be zero before the first use. The split count changes rounding only, never which keys are seen.
  * fp16/bf16 q and cache of the same dtype with head_dim 64 or 128 and 16-byte aligned
  * operands run on MFMA with the reference's tl.dot numerics (fp32 scores, probabilities
  * rounded to the cache dtype for P.V); every other case computes in fp32. Context lengths

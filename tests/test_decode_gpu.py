@@ -339,3 +339,60 @@ def test_decode_graph_capture_replays_match_eager():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager), f"replay {i}"
+
+
+def _shapes():
+    out = []
+    for i, (batch, hq, hkv, d, dtype, splits) in enumerate([
+            (9, 32, 8, 128, torch.bfloat16, 3), (1200, 14, 2, 64, torch.float16, 2), (5, 8, 2, 64, torch.float32, 4),
+            (70, 16, 4, 128, torch.bfloat16, 16), (9, 32, 8, 128, torch.bfloat16, 3)]):
+        ctx = _ragged(batch, 200 if batch > 1000 else 900, 16, seed=20 + i)
+        args = _to_dev(*gen.decode_inputs(ctx, hq, hkv, d, 16, dtype, seed=20 + i))
+        out.append((args, d ** -0.5, splits))
+    return out
+
+
+def test_decode_shapes_take_turns_on_one_workspace(monkeypatch):
+    """Calls of different shapes share the stream's workspace (partials at its start, counters at
+    its end; 16800 (sequence, head) rows outgrow the first counters): every one gives the bits of
+    a workspace of its own, also when the shapes come round again."""
+    from emberserve_amd import _scratch
+    from emberserve_amd import paged_decode as pd
+    calls, want = _shapes(), []
+    for args, scale, splits in calls:
+        monkeypatch.setattr(pd, "_SCRATCH", _scratch.SharedScratch("t"))
+        want.append(paged_attention_decode(*args, scale, num_splits=splits))
+    monkeypatch.setattr(pd, "_SCRATCH", _scratch.SharedScratch("t"))
+    for _ in range(2):
+        for (args, scale, splits), w in zip(calls, want):
+            _say(f"shared workspace B={args[0].shape[0]} splits={splits}")
+            assert torch.equal(paged_attention_decode(*args, scale, num_splits=splits), w)
+    assert len(pd._SCRATCH._bufs) == 1 and _lib.read_errors() == 0
+
+
+def test_decode_graphs_of_several_shapes_replay_in_any_order(monkeypatch):
+    """Two graphs captured on a stream that no eager call has used, the larger shape first: each
+    fills its own counters, so the second may be replayed before the first, and eager calls run
+    between the replays."""
+    from emberserve_amd import _scratch
+    from emberserve_amd import paged_decode as pd
+    calls = [_shapes()[i] for i in (3, 0)]
+    want = [paged_attention_decode(*args, scale, num_splits=splits) for args, scale, splits in calls]
+    monkeypatch.setattr(pd, "_SCRATCH", _scratch.SharedScratch("t"))
+    side, graphs = torch.cuda.Stream(), []
+    torch.cuda.synchronize()
+    for args, scale, splits in calls:
+        out = torch.empty_like(args[0])
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=side):
+            for _ in range(2):
+                paged_attention_decode(*args, scale, num_splits=splits, out=out)
+        graphs.append((g, out))
+    for i in range(3):
+        for (g, out), w, (args, scale, splits) in reversed(list(zip(graphs, want, calls))):
+            out.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, w), f"replay {i}"
+            assert torch.equal(paged_attention_decode(*args, scale, num_splits=splits), w)
+    assert _lib.read_errors() == 0
