@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import threading
+import warnings
 from pathlib import Path
 
 import torch
@@ -143,18 +144,25 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
         if got != ABI_VERSION:
             raise RuntimeError(f"emberserve_amd: {p} has ABI version {got}, expected {ABI_VERSION}; rebuild it")
         if path is None:
-            try:
-                from . import _fast
-            except ImportError as e:
-                raise RuntimeError(f"emberserve_amd: _fast.so is not built ({e}); run `python -m "
-                                   "emberserve_amd.build`") from None
-            if _fast.ABI_VERSION != ABI_VERSION:
-                raise RuntimeError(f"emberserve_amd: _fast.so has ABI version {_fast.ABI_VERSION}, expected "
-                                   f"{ABI_VERSION}; rebuild it")
-            _fast.bind({name: ctypes.cast(getattr(lib, name), _p).value for name in SIGNATURES})
-            fast.__dict__.update({k: v for k, v in vars(_fast).items() if not k.startswith("__")})
+            _load_fast(lib)
             _lib = lib
         return lib
+
+
+def _load_fast(lib: ctypes.CDLL) -> None:
+    """Fills `fast` from _fast.so. Without the extension every call takes the Python wrappers: the
+    same kernels and results, at about 16 us of host time a launch instead of 5."""
+    try:
+        from . import _fast
+    except ImportError as e:
+        warnings.warn(f"emberserve_amd: no native host path ({e}); `python -m emberserve_amd.build` builds it where "
+                      "a C++ compiler and torch's and Python's headers are installed", RuntimeWarning, stacklevel=3)
+        return
+    if _fast.ABI_VERSION != ABI_VERSION:
+        raise RuntimeError(f"emberserve_amd: _fast.so has ABI version {_fast.ABI_VERSION}, expected "
+                           f"{ABI_VERSION}; rebuild it")
+    _fast.bind({name: ctypes.cast(getattr(lib, name), _p).value for name in SIGNATURES})
+    fast.__dict__.update({k: v for k, v in vars(_fast).items() if not k.startswith("__")})
 
 
 def dtype_tag(dtype: torch.dtype) -> int:

@@ -15,6 +15,7 @@ import shutil
 import subprocess
 import sys
 import sysconfig
+import warnings
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
@@ -52,15 +53,20 @@ def _compile(src: Path, obj: Path) -> None:
 
 
 def _build_fast() -> None:
-    """Compiles csrc/fast_ops.cpp into _fast.so."""
+    """Compiles csrc/fast_ops.cpp into _fast.so. Where a C++ compiler or the headers are not
+    installed there is no native host path (nor a stale one): the library does without it."""
     import torch
 
     cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
-    if cxx is None:
-        raise RuntimeError("no C++ compiler found (set CXX)")
     rocm = Path(hipcc()).resolve().parent.parent
     inc = Path(torch.__file__).resolve().parent / "include"
     lib = inc.parent / "lib"
+    headers = [Path(sysconfig.get_paths()["include"]) / "Python.h", inc / "torch/csrc/autograd/python_variable.h"]
+    missing = ["a C++ compiler (set CXX)"] * (cxx is None) + [str(h) for h in headers if not h.exists()]
+    if missing:
+        FAST_PATH.unlink(missing_ok=True)
+        warnings.warn(f"emberserve_amd: _fast.so is not built, {' and '.join(missing)} not found", RuntimeWarning)
+        return
     tmp = FAST_PATH.with_suffix(".so.tmp")
     cmd = [*cxx.split(), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{inc}",

@@ -6,13 +6,15 @@ the others (which the wrappers convert, refuse or run eagerly)."""
 from __future__ import annotations
 
 import ctypes
+import os
 import subprocess
 import sys
+from pathlib import Path
 
 import pytest
 import torch
 
-from emberserve_amd import _lib, ops
+from emberserve_amd import _lib, build, ops
 from emberserve_amd.mla_decode import mla_decode
 from emberserve_amd.paged_decode import paged_attention_decode
 from emberserve_amd.rope import RotaryEmbedding
@@ -54,6 +56,34 @@ def test_extension_is_imported_by_load():
             "assert 'emberserve_amd._fast' not in sys.modules and _lib.fast.rmsnorm(1) is None\n"
             "_lib.load(); assert 'rmsnorm' in vars(_lib.fast)")
     subprocess.run([sys.executable, "-c", code], check=True, timeout=300)
+
+
+def test_the_library_loads_without_the_extension(tmp_path):
+    """A tree built without a host compiler: the package warns once and runs the Python wrappers."""
+    pkg = tmp_path / "emberserve_amd"
+    pkg.mkdir()
+    for f in Path(_lib.__file__).parent.iterdir():
+        if f.name not in ("_fast.so", "__pycache__"):
+            (pkg / f.name).symlink_to(f)
+    code = ("import warnings, torch; from emberserve_amd import _lib, ops\n"
+            "with warnings.catch_warnings(record=True) as w:\n"
+            "    warnings.simplefilter('always'); _lib.load(); _lib.load()\n"
+            "assert ['native host path' in str(x.message) for x in w].count(True) == 1, w\n"
+            "assert _lib.__file__.startswith(%r) and _lib.fast.rmsnorm(1) is None\n"
+            "x = torch.randn(2, 8); assert torch.equal(ops.silu_and_mul(x), ops.silu_and_mul_torch(x))" % str(tmp_path))
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=300, cwd=tmp_path,
+                   env={**os.environ, "PYTHONPATH": ""})
+
+
+def test_build_without_a_compiler_leaves_no_extension(tmp_path, monkeypatch):
+    monkeypatch.delenv("CXX", raising=False)
+    monkeypatch.setattr(build.shutil, "which", lambda name: None)
+    monkeypatch.setattr(build, "hipcc", lambda: "/opt/rocm/bin/hipcc")
+    monkeypatch.setattr(build, "FAST_PATH", tmp_path / "_fast.so")
+    (tmp_path / "_fast.so").write_bytes(b"stale")
+    with pytest.warns(RuntimeWarning, match="compiler"):
+        build._build_fast()
+    assert not (tmp_path / "_fast.so").exists()
 
 
 gpu = pytest.mark.gpu
