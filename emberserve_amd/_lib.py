@@ -15,7 +15,7 @@ import torch
 from torch.compiler import is_dynamo_compiling as tracing  # noqa: F401  (for the callers of `fast`)
 
 LIB_PATH = Path(__file__).resolve().parent / "libember_ops.so"
-ABI_VERSION = 19
+ABI_VERSION = 20
 
 F32, F16, BF16 = 0, 1, 2
 ERR_EMBED_ID = 1
@@ -75,6 +75,9 @@ SIGNATURES: dict[str, list] = {
     "ember_paged_decode": [_p, _i64, _i64, _i32, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                            _i64, _i32, _p, _i64, _i64, _p, _i64, _i64, _f32, _i64, _i32, _p, _i64, _p, _i64,
                            _i64, _p],
+    "ember_paged_decode_shared": [_p, _i64, _i64, _i32, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
+                                  _i64, _i32, _p, _i64, _i64, _p, _i64, _i64, _f32, _i64, _i32, _p, _i64, _p, _i64,
+                                  _i64, _p],
     "ember_paged_decode_noalloc_max_bytes": [],
     "ember_paged_decode_noalloc": [_p, _i64, _i64, _i32, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                    _i64, _i64, _i32, _p, _i64, _i64, _p, _i64, _i64, _f32, _i64, _i32, _p, _i64,

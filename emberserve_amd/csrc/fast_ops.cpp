@@ -51,7 +51,7 @@ Entry g_entry[kEntries] = {
     {"ember_rmsnorm", nullptr}, {"ember_fused_add_rmsnorm", nullptr}, {"ember_rope", nullptr},
     {"ember_silu_and_mul", nullptr}, {"ember_embedding", nullptr}, {"ember_qk_norm_rope", nullptr},
     {"ember_mla_latent_rope", nullptr}, {"ember_rope_kv_cache", nullptr}, {"ember_mla_latent_rope_cache", nullptr},
-    {"ember_paged_decode", nullptr}, {"ember_mla_decode", nullptr}, {"ember_status_string", nullptr}};
+    {"ember_paged_decode_shared", nullptr}, {"ember_mla_decode", nullptr}, {"ember_status_string", nullptr}};
 bool g_bound = false;
 
 #define ENTRY(i, f) reinterpret_cast<decltype(&f)>(g_entry[i].fn)
@@ -530,7 +530,7 @@ PyObject* paged_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   at::Tensor out = at::empty(q->sizes(), q->options());
   void* s = c.stream();
   const int st = launch([&] {
-    return ENTRY(kPagedDecode, ember_paged_decode)(
+    return ENTRY(kPagedDecode, ember_paged_decode_shared)(
         q->data_ptr(), q->stride(0), q->stride(1), tag, kc->data_ptr(), vc->data_ptr(), kc->size(0), bs, hk, d,
         kc->stride(0), kc->stride(1), kc->stride(2), vc->stride(0), vc->stride(1), vc->stride(2), ctag,
         static_cast<const int32_t*>(bt->data_ptr()), bt->stride(0), bt->size(1),
@@ -590,7 +590,7 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_fast", nullptr, -1, kMethods, nu
 PyMODINIT_FUNC PyInit__fast(void) {
   PyObject* m = PyModule_Create(&kModule);
   // the ABI version (ember_abi_version) of the header this was compiled against
-  if (m != nullptr && PyModule_AddIntConstant(m, "ABI_VERSION", 19) != 0) {
+  if (m != nullptr && PyModule_AddIntConstant(m, "ABI_VERSION", 20) != 0) {
     Py_DECREF(m);
     return nullptr;
   }

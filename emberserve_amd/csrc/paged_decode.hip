@@ -791,9 +791,8 @@ int64_t ember_paged_decode_workspace_bytes(int64_t num_seqs, int64_t num_heads, 
 namespace ember {
 namespace {
 
-// ember_paged_decode's body. The arrival counters are the workspace's last words, whatever part
-// of it the call's partials need, so that calls of different shapes on one buffer find them at
-// zero; `counters` (when non-null) replaces them (the no-allocation entry point's fixed place).
+// The entry points' body. The arrival counters follow the partials, unless `counters` (non-null)
+// gives them another place.
 int paged_decode_core(const void* q, int64_t q_seq_stride, int64_t q_head_stride, int q_dtype,
                       const void* k_cache, const void* v_cache, int64_t num_blocks, int64_t block_size,
                       int64_t num_kv_heads, int64_t head_dim, int64_t k_block_stride, int64_t k_slot_stride,
@@ -856,11 +855,7 @@ int paged_decode_core(const void* q, int64_t q_seq_stride, int64_t q_head_stride
     a.part_m = ws;
     a.part_l = ws + rows;
     a.part_o = ws + 2 * rows;
-    const int64_t counter_bytes = need - rows * (head_dim + 2) * int64_t(sizeof(float));
-    a.counters = counters != nullptr
-                     ? counters
-                     : reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) +
-                                                   ((workspace_bytes - counter_bytes) & ~int64_t(3)));
+    a.counters = counters != nullptr ? counters : reinterpret_cast<uint32_t*>(ws + rows * (head_dim + 2));
   }
   a.err = err;
   hipStream_t st = static_cast<hipStream_t>(stream);
@@ -928,6 +923,28 @@ int ember_paged_decode(const void* q, int64_t q_seq_stride, int64_t q_head_strid
                            v_slot_stride, v_head_stride, cache_dtype, block_tables, block_table_stride, max_blocks,
                            context_lens, num_seqs, num_heads, scale, num_splits, flags, workspace, workspace_bytes,
                            nullptr, out, out_seq_stride, out_head_stride, stream);
+}
+
+int ember_paged_decode_shared(const void* q, int64_t q_seq_stride, int64_t q_head_stride, int q_dtype,
+                              const void* k_cache, const void* v_cache, int64_t num_blocks, int64_t block_size,
+                              int64_t num_kv_heads, int64_t head_dim, int64_t k_block_stride, int64_t k_slot_stride,
+                              int64_t k_head_stride, int64_t v_block_stride, int64_t v_slot_stride,
+                              int64_t v_head_stride, int cache_dtype, const int32_t* block_tables,
+                              int64_t block_table_stride, int64_t max_blocks, const int32_t* context_lens,
+                              int64_t num_seqs, int64_t num_heads, float scale, int64_t num_splits, int flags,
+                              void* workspace, int64_t workspace_bytes, void* out, int64_t out_seq_stride,
+                              int64_t out_head_stride, void* stream) {
+  if (num_seqs < 0 || num_heads < 0) return EMBER_EINVAL;
+  const int64_t counter_bytes = (num_seqs * num_heads * int64_t(sizeof(uint32_t)) + 15) / 16 * 16;
+  uint32_t* counters = workspace == nullptr || workspace_bytes < counter_bytes
+                           ? nullptr
+                           : reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) +
+                                                         ((workspace_bytes - counter_bytes) & ~int64_t(3)));
+  return paged_decode_core(q, q_seq_stride, q_head_stride, q_dtype, k_cache, v_cache, num_blocks, block_size,
+                           num_kv_heads, head_dim, k_block_stride, k_slot_stride, k_head_stride, v_block_stride,
+                           v_slot_stride, v_head_stride, cache_dtype, block_tables, block_table_stride, max_blocks,
+                           context_lens, num_seqs, num_heads, scale, num_splits, flags, workspace, workspace_bytes,
+                           counters, out, out_seq_stride, out_head_stride, stream);
 }
 
 }  // extern "C"

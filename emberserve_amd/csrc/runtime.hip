@@ -45,7 +45,7 @@ __host__ int device_cu_count() {
 
 extern "C" {
 
-int ember_abi_version(void) { return 19; }
+int ember_abi_version(void) { return 20; }
 
 const char* ember_status_string(int status) {
   switch (status) {

@@ -128,8 +128,8 @@ _SCRATCH = SharedScratch("paged_attention_decode")
 
 
 def _workspace(num_splits: int, batch: int, num_heads: int, head_dim: int, device: torch.device) -> Tensor:
-    """The workspace of a call: ember_paged_decode_workspace_bytes of partials and, at the
-    buffer's end, counters."""
+    """The workspace of a call, for ember_paged_decode_shared: partials at the buffer's start,
+    counters at its end."""
     rows = batch * num_heads
     return _SCRATCH.get(num_splits * rows * (head_dim + 2) * 4, round_up(rows * 4, 16), device)
 
@@ -210,7 +210,7 @@ def paged_attention_decode(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_ta
     if num_splits > 1:
         ws = _workspace(num_splits, B, H, D, q.device)
     flags = _lib.DECODE_FP32 if variant == "sum" else 0
-    _launch("ember_paged_decode", _lib.load().ember_paged_decode, q.device,
+    _launch("ember_paged_decode", _lib.load().ember_paged_decode_shared, q.device,
             q.data_ptr(), q.stride(0), q.stride(1), _lib.dtype_tag(q.dtype),
             k_cache.data_ptr(), v_cache.data_ptr(), num_blocks, block_size, Hkv, D,
             k_cache.stride(0), k_cache.stride(1), k_cache.stride(2),

@@ -301,11 +301,10 @@ int64_t ember_paged_decode_workspace_bytes(int64_t num_seqs, int64_t num_heads, 
  * sequence's context is cut into num_splits key ranges whose partial results are merged by
  * the last split to finish (or a second kernel) through `workspace`
  * (at least ember_paged_decode_workspace_bytes bytes, 16-byte aligned, zero-filled before its
- * first use; every call leaves it ready for the next, and calls that overlap on one workspace
- * race). The partials are at its start and the counters are its last num_seqs x num_heads
- * words (rounded up to 16 bytes), so calls of different shapes may take turns on one larger
- * workspace of a fixed size as long as no call's partials reach another's counters; then only
- * the counters have to be zero before the first use. The split count changes rounding only, never which keys are seen.
+ * first use; every call of the same shape leaves it ready for the next, and calls that overlap
+ * on one workspace race). The partials are at its start, the counters (num_seqs x num_heads
+ * words, rounded up to 16 bytes) behind them. The split count changes rounding only, never
+ * which keys are seen.
  * fp16/bf16 q and cache of the same dtype with head_dim 64 or 128 and 16-byte aligned
  * operands run on MFMA with the reference's tl.dot numerics (fp32 scores, probabilities
  * rounded to the cache dtype for P.V); every other case computes in fp32. Context lengths
@@ -324,6 +323,21 @@ int ember_paged_decode(const void* q, int64_t q_seq_stride, int64_t q_head_strid
                        const int32_t* context_lens, int64_t num_seqs, int64_t num_heads, float scale,
                        int64_t num_splits, int flags, void* workspace, int64_t workspace_bytes,
                        void* out, int64_t out_seq_stride, int64_t out_head_stride, void* stream);
+
+/* ember_paged_decode with the counters as the last num_seqs x num_heads words (rounded up to 16
+ * bytes) of the workspace_bytes given: calls of different shapes may take turns on one workspace
+ * of a fixed size, as long as no call's partials reach another's counters. Only the counters have
+ * to be zero before its first use. Arguments and results are ember_paged_decode's. */
+int ember_paged_decode_shared(const void* q, int64_t q_seq_stride, int64_t q_head_stride, int q_dtype,
+                              const void* k_cache, const void* v_cache, int64_t num_blocks, int64_t block_size,
+                              int64_t num_kv_heads, int64_t head_dim,
+                              int64_t k_block_stride, int64_t k_slot_stride, int64_t k_head_stride,
+                              int64_t v_block_stride, int64_t v_slot_stride, int64_t v_head_stride,
+                              int cache_dtype,
+                              const int32_t* block_tables, int64_t block_table_stride, int64_t max_blocks,
+                              const int32_t* context_lens, int64_t num_seqs, int64_t num_heads, float scale,
+                              int64_t num_splits, int flags, void* workspace, int64_t workspace_bytes,
+                              void* out, int64_t out_seq_stride, int64_t out_head_stride, void* stream);
 
 /* ember_paged_decode without a workspace argument, for callers that cannot allocate (code
  * under HIP graph capture that may not call hipMalloc, tight serving loops, harnesses that

@@ -370,6 +370,35 @@ def test_decode_shapes_take_turns_on_one_workspace(monkeypatch):
     assert len(pd._SCRATCH._bufs) == 1 and _lib.read_errors() == 0
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_decode_entry_points_keep_their_counters_apart(dtype):
+    """Over a workspace larger than the call's need, ember_paged_decode's counters follow its
+    partials (what lies behind the needed bytes may hold anything) and
+    ember_paged_decode_shared's are the last words (the rest may hold anything)."""
+    lib, splits = _lib.load(), 4
+    q, kc, vc, bt, cl = _to_dev(*gen.decode_inputs([5, 700, 33], 32, 8, 128, 16, dtype, seed=31))
+    rows = q.shape[0] * q.shape[1]
+    need = lib.ember_paged_decode_workspace_bytes(q.shape[0], q.shape[1], 128, splits)
+    args = (q.data_ptr(), q.stride(0), q.stride(1), _lib.dtype_tag(dtype), kc.data_ptr(), vc.data_ptr(), kc.shape[0],
+            16, 8, 128, kc.stride(0), kc.stride(1), kc.stride(2), vc.stride(0), vc.stride(1), vc.stride(2),
+            _lib.dtype_tag(dtype), bt.data_ptr(), bt.stride(0), bt.shape[1], cl.data_ptr(), *q.shape[:2],
+            float(128 ** -0.5), splits, 0)
+    outs = []
+    for fn, size, zero in ((lib.ember_paged_decode, need, slice(0, need // 4)),
+                           (lib.ember_paged_decode, 2 * need, slice(0, need // 4)),
+                           (lib.ember_paged_decode_shared, 2 * need, slice(2 * need // 4 - rows, None))):
+        ws = torch.full((size // 4,), 77, dtype=torch.int32, device=DEV)
+        ws[zero] = 0
+        for _ in range(2):
+            out = torch.full_like(q, float("nan"))
+            _say(f"{fn.__name__} {dtype} workspace {size} of {need}")
+            assert fn(*args, ws.data_ptr(), size, out.data_ptr(), out.stride(0), out.stride(1),
+                      torch.cuda.current_stream().cuda_stream) == 0
+            outs.append(out)
+    assert all(torch.equal(o, outs[0]) for o in outs) and not bool(outs[0].isnan().any())
+    assert _lib.read_errors() == 0
+
+
 def test_decode_graphs_of_several_shapes_replay_in_any_order(monkeypatch):
     """Two graphs captured on a stream that no eager call has used, the larger shape first: each
     fills its own counters, so the second may be replayed before the first, and eager calls run

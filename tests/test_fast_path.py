@@ -244,7 +244,7 @@ def test_a_failed_launch_is_raised_and_not_run_again(monkeypatch):
     from emberserve_amd import _fast
     lib, st = _lib.load(), 3
     real = {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _lib.SIGNATURES}
-    names = ("ember_rope", "ember_rope_kv_cache", "ember_rmsnorm", "ember_paged_decode")
+    names = ("ember_rope", "ember_rope_kv_cache", "ember_rmsnorm", "ember_paged_decode_shared")
     stubs = [ctypes.CFUNCTYPE(ctypes.c_int, *_lib.SIGNATURES[n])(lambda *a: st) for n in names]
     again = []
     for name in ("rope_hip", "rope_kv_cache_hip", "rmsnorm_hip"):
@@ -257,7 +257,7 @@ def test_a_failed_launch_is_raised_and_not_run_again(monkeypatch):
     calls = {"rope": lambda: ops.rope(q, k, cos, sin, pos),
              "rope_kv_cache": lambda: ops.rope_kv_cache(q, k, v, cos, sin, pos, pos, *caches),
              "rmsnorm": lambda: ops.rmsnorm(q.view(3, -1), _rand(256), 1e-6),
-             "paged_decode": lambda: paged_attention_decode(*dec, 0.1)}
+             "paged_decode_shared": lambda: paged_attention_decode(*dec, 0.1)}
     _fast.bind({**real, **{n: ctypes.cast(s, ctypes.c_void_p).value for n, s in zip(names, stubs)}})
     try:
         for what, call in calls.items():
