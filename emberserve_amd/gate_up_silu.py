@@ -241,7 +241,13 @@ def packed_gemm_default(tokens: int, hidden: int, inter: int, device: torch.devi
     128: 46 | 50, 160: 51 | 55, 200: 60 | 63, 256: 63 | 65, 300: 70 | 76, 512: 90 | 91, but 2048: 317 | 301;
     Qwen2.5-7B 64: 51 | 62, 128: 56 | 70, 256: 80 | 82, but 600: 188 | 172; Qwen2.5-0.5B (H 896)
     100: 9.3 | 13, 1024: 27 | 37, 8192: 161 | 199."""
-    return hidden <= 1024 or -(-tokens // 256) * -(-inter // 128) <= num_sms(device)
+    return _gemm_takes(hidden, inter) and (hidden <= 1024
+                                           or -(-tokens // 256) * -(-inter // 128) <= num_sms(device))
+
+
+def _gemm_takes(hidden: int, inter: int) -> bool:
+    """The packed GEMM's own limits; the decode kernel and the pair go beyond them."""
+    return hidden <= 1 << 20 and inter <= 1 << 28
 
 
 def gate_up_silu(x: Tensor, weight: Tensor | None, *, num_workgroups: int | None = None,
@@ -258,7 +264,8 @@ def gate_up_silu(x: Tensor, weight: Tensor | None, *, num_workgroups: int | None
             raise ValueError("gate_up_silu: weight None needs the packed weight")
         if fused is False:
             raise ValueError("gate_up_silu: the unfused pair needs the unpacked weight")
-        limit = PACKED_FUSED_TOKENS if num_workgroups is None else PACKED_MAX_TOKENS
+        gemm = num_workgroups is None and _gemm_takes(packed.hidden, packed.inter)
+        limit = PACKED_FUSED_TOKENS if gemm else PACKED_MAX_TOKENS
         if x.reshape(-1, packed.hidden).shape[0] > limit:
             return gate_up_silu_gemm_packed(x, packed)
         return _packed_decode(x, packed, num_workgroups)

@@ -330,6 +330,22 @@ def test_gate_up_silu_cpu_path_is_the_unfused_pair():
         gate_up_silu(x, w[:95])
 
 
+@pytest.mark.parametrize("hidden,inter,gemm", [(256, 256, True), (1 << 20, 64, True), ((1 << 20) + 64, 64, False),
+                                               (64, (1 << 28) + 64, False)])
+def test_gate_up_silu_sizes_past_the_packed_gemm_keep_their_kernels(monkeypatch, hidden, inter, gemm):
+    """33 to 64 tokens over the packed copy alone, and the default beside the unpacked weight: sizes
+    that the packed GEMM refuses stay with the decode kernel and with the pair."""
+    from emberserve_amd import gate_up_silu as mod
+    monkeypatch.setattr(mod, "num_sms", lambda device: 1 << 24)
+    monkeypatch.setattr(mod, "gate_up_silu_gemm_packed", lambda x, packed: "gemm")
+    monkeypatch.setattr(mod, "_packed_decode", lambda x, packed, n: "decode")
+    packed = mod.PackedGateUp(torch.empty(0, dtype=torch.bfloat16), hidden, inter, 7)
+    x = torch.empty(48, hidden, dtype=torch.bfloat16, device="meta")
+    assert mod.gate_up_silu(x, None, packed=packed) == ("gemm" if gemm else "decode")
+    assert mod.gate_up_silu(x[:32], None, packed=packed) == "decode"
+    assert mod.packed_gemm_default(48, hidden, inter, torch.device("cpu")) == gemm
+
+
 def test_gate_up_silu_workspace_plan():
     """Units are (64-column slab, 64-k step) pairs in slab-major order; workgroup b runs
     units [floor(b total / G), floor((b + 1) total / G)). The workspace holds, per slab, one
