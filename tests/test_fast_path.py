@@ -143,8 +143,10 @@ def test_head_ops_equal_the_python_wrappers(dtype, hq, hk, d):
             w = (qw, kw) if norm else (None, None)
             got = fast.rope_kv_cache(*a, cos, sin, pos, slots, caches[0], caches[1], *w, 1e-6)
             want = ops.rope_kv_cache_hip(*b, cos, sin, pos, slots, caches[2], caches[3], *w, 1e-6)
-            if got is None:  # operands the fused kernel refuses: the wrappers run the unfused pair
+            if d == 96:  # heads that the fused kernel refuses: the wrappers run the unfused pair
+                assert got is None
                 got = ops.rope_kv_cache_hip(*a, cos, sin, pos, slots, caches[0], caches[1], *w, 1e-6)
+            assert got[0] is a[0] and got[1] is a[1]
             _same(got, want, "rope_kv_cache")
             assert torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3])
 
@@ -192,8 +194,15 @@ def test_decode_equals_the_python_wrapper(monkeypatch):
         _same(got, want, "paged_decode")
     q, lat, bt, cl = (t.to(DEV) for t in gen.mla_decode_inputs([5, 700, 33], 16, 512, 64, 16, torch.bfloat16, seed=3))
     want = mla_decode(q, lat, bt, cl, 0.07, 512, out=torch.empty(3, 16, 512, dtype=q.dtype, device=DEV))
-    _same(mla_decode(q, lat, bt, cl, 0.07, 512), want, "mla_decode")
-    _same(mla_decode((q[..., :512].contiguous(), q[..., 512:].contiguous()), lat, bt, cl, 0.07, 512), want, "pair")
+    real = fast.mla_decode
+    for operand, what in ((q, "mla_decode"), ((q[..., :512].contiguous(), q[..., 512:].contiguous()), "pair")):
+        calls = []
+        monkeypatch.setattr(_lib, "fast", type("F", (), {"mla_decode": staticmethod(
+            lambda *a: calls.append(real(*a)) or calls[-1])}))
+        got = mla_decode(operand, lat, bt, cl, 0.07, 512)
+        monkeypatch.undo()
+        assert calls[0] is got
+        _same(got, want, what)
     assert _lib.read_errors() == 0
 
 
