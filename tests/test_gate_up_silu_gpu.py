@@ -394,6 +394,7 @@ def test_fused_true_past_64_tokens_runs_the_gemm():
     x = (torch.randn(100, 512, generator=g) * 0.5).to(torch.bfloat16).to(DEV)
     assert torch.equal(gate_up_silu(x, w48, fused=True), gate_up_silu_torch(x, w48))
 
+
 @pytest.mark.parametrize("tokens", [16, 48, 64])
 def test_packed_only_keeps_the_given_workgroups(tokens):
     """With the packed copy alone, num_workgroups means the decode kernel up to its 64 tokens:
@@ -417,3 +418,20 @@ def test_overlapping_rows_run_the_pair():
     for view in (dx[:1].expand(48, 256), dx.view(-1).as_strided((32 + 1, 256), (8, 1))):
         _say(f"overlapping rows, strides {tuple(view.stride())}")
         assert torch.equal(gate_up_silu(view, dw, packed=packed), gate_up_silu_torch(view, dw))
+
+
+@pytest.mark.parametrize("tokens,stride", [(256, 1 << 22), (3, (1 << 22) + 8)])
+def test_gemm_packed_far_rows(tokens, stride):
+    """The packed GEMM addresses a tile's rows by 32-bit byte offsets: a whole 256-token tile at the
+    largest stride of that form (255 x 2^23 bytes, just under 2^31), and rows farther apart, which
+    go one token a launch. The bits of contiguous rows."""
+    from emberserve_amd.gate_up_silu import gate_up_silu_gemm_packed, pack_gate_up_weight
+    _say(f"packed gemm T={tokens} x row stride {stride}")
+    x, w = gen.gate_up_inputs(tokens, 256, 256, torch.bfloat16, seed=33)
+    dx, packed = x.to(DEV), pack_gate_up_weight(w.to(DEV))
+    far = torch.empty((tokens - 1) * stride + 256, dtype=x.dtype, device=DEV).as_strided((tokens, 256), (stride, 1))
+    far.copy_(dx)
+    for tile in (None, 64):
+        want = gate_up_silu_gemm_packed(dx, packed, column_tile=tile)
+        got = gate_up_silu_gemm_packed(far, packed, column_tile=tile)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), tile

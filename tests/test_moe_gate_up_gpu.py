@@ -359,3 +359,32 @@ def test_moe_gemm_block_rows_rule():
     assert [rule(a, 64, 1408, 256, False) for a in (1023, 1024, 12287, 12288)] == [0, 128, 128, 256]
     assert [rule(a, 128, 768, 256, True) for a in (1279, 1280, 4096, 24575, 24576)] == [0, 64, 128, 128, 256]
     assert [rule(a, 8, 1408, 256, p) for a in (160, 1535, 1536) for p in (False, True)] == [0, 0, 0, 0, 128, 128]
+
+
+@pytest.mark.parametrize("below", [True, False])
+def test_packed_moe_gemm_far_rows(monkeypatch, below):
+    """Packed experts' 64- and 128-row blocks address x rows by 32-bit offsets while x spans less than
+    2^29 elements; from there the 64-row ones are refused (and not chosen) and the 128-row ones run
+    with both operands in LDS. The bits of contiguous rows either way."""
+    import emberserve_amd.moe as moe_mod
+
+    n, experts, k, hidden, inter = 1024, 224, 3, 256, 128
+    stride = (1 << 29) // n - (8 if below else 0)
+    print(f"moe packed gemm x row stride {stride}", flush=True)
+    g = torch.Generator().manual_seed(34)
+    x = (torch.randn(n, hidden, generator=g) * 0.5).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(experts, 2 * inter, hidden, generator=g) / 16).to(torch.bfloat16).to(DEV)
+    ids = torch.stack([torch.randperm(experts, generator=g)[:k] for _ in range(n)]).to(DEV)
+    far = torch.empty((n - 1) * stride + hidden, dtype=x.dtype, device=DEV).as_strided((n, hidden), (stride, 1))
+    far.copy_(x)
+    packed = pack_moe_gate_up_weight(w)
+    si, be, nv = moe_align(ids, experts)
+    want = moe_gate_up_silu(x, w, si, be, nv, k, num_splits=1)
+    rows64, calls = moe_mod._moe_gemm_rows64, []
+    monkeypatch.setattr(moe_mod, "_moe_gemm_rows64", lambda *a: calls.append(1) or rows64(*a))
+    assert torch.equal(fused_moe_gate_up(far, ids, w, packed=packed), want)
+    assert len(calls) == below
+    assert torch.equal(moe_gate_up_silu_gemm(far, None, ids, block_rows=128, packed=packed), want)
+    if not below:
+        with pytest.raises(RuntimeError, match="status 5"):  # EMBER_ETOOBIG
+            rows64(far, ids, packed)
