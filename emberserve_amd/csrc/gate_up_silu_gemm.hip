@@ -720,11 +720,16 @@ int launch_frag(const GemmArgs& a, hipStream_t st) {
   return launch_status();
 }
 
-// A tile's workgroup takes about as long as the rows it streams, BM x rows and 2 x columns
-// weight rows per k, whatever their split (us per round of tiles at H = 4096; rows: 224 41-46,
-// 256 45-50, 288 53-56, 320 60-63, 352 55-61, 384 56-72, 448 70-88, 512 87-111): the tile with
-// the fewest rows in all rounds, the smaller on a tie. The
-// 192-token tiles: Qwen3-8B 160 tokens 60 -> 51 us, 300: 89 -> 70, 700: 164 -> 134.
+// A tile's workgroup takes about as long as the rows it needs, BM x rows and 2 x columns weight
+// rows per k: the tile with the fewest rows in all rounds, the smaller on a tie. Measured (bf16,
+// us, one round at H = 4096; rows: 224 41-46, 256 45-50, 288 45-56, 320 49-63, 352 55-68, 384 59-73,
+// 416 78-82, 448 70-91, 512 84-112): not a strict order. 80-column tiles of 192 and 256 tokens take
+// longer than 96-column ones, 128 x 96 longer than 192 x 64. Still the pick is the fastest of the
+// sixteen tiles, or within 2%, at 64 to 700 tokens of Qwen3-8B, 64 to 600 of Qwen2.5-7B and 100 to
+// 1024 of Qwen2.5-0.5B (2000: 48.2 against 45.0 at 128 x 64). BM + 4 x columns, the rows that the
+// loads issue (both token groups load the weights, the second from L1), picks worse: Qwen3-8B 200
+// tokens 65 against 60, 256: 68 against 63, 600: 138 against 134, and nowhere better.
+// The 192-token tiles: Qwen3-8B 160 tokens 59 -> 53 us, 300: 87 -> 70, 700: 160 -> 141.
 void frag_pick_tile(int64_t tokens, int64_t inter, int64_t& token_tile, int64_t& column_tile) {
   const int64_t ncu = std::max(1, device_cu_count());
   int64_t best = INT64_MAX;
