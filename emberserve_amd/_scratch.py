@@ -79,12 +79,14 @@ class _Buffer(NamedTuple):
 
 class SharedScratch(_Verified):
     """One workspace per (thread, device, current stream) for calls of every shape, for an entry
-    point that keeps its partials at the workspace's start and its counters at the end (paged
-    decode). Its split count varies with the batch, so that a workspace for each shape, kept for
-    good, came to 1.3 GB over batches of 1 to 256 (32q/8kv x 128, 8192-key tables), against 40 MB
-    here. The partials' part at least doubles when it grows. An outgrown buffer is kept, because a
-    captured graph may hold its address: all of a stream's together are at most four times its
-    largest call's need.
+    point that keeps its partials at the workspace's start and its counters at the end
+    (ember_paged_decode_shared). Per thread, because a call may be two launches (the fp32 kernel and
+    its merge), between which another thread's on the same stream would overwrite its partials. The
+    split count varies with the batch, so that a workspace for each shape, kept for good, came to
+    1.3 GB over batches of 1 to 256 (32q/8kv x 128, 8192-key tables), against 40 MB here. The
+    partials' part at least doubles when it grows. An outgrown buffer is kept, because a captured
+    graph may hold its address: all of a stream's together are at most four times its largest
+    call's need.
 
     A call captured where no eager call has left a large enough workspace gets one that belongs to
     that capture: its memory is the graph's own, and the zero fill of its counters is recorded in

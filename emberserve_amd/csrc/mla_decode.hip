@@ -214,7 +214,8 @@ __device__ __forceinline__ int small_ceil_div(int x, int y) {
 // With it, all into parts of one size, the least of five that fits the units: per =
 // ceil(tiles / (units - k nseq / 4)), k = 0 .. 4 (k = 4 always fits: a context takes at most
 // floor(tiles / per) + 1), so the long contexts of a ragged batch use the units that the short ones
-// leave. Every context takes one unit at least.
+// leave; a sequence's parts, and so its rounding, then depend on the batch's other contexts. Every
+// context takes one unit at least.
 struct SplitPlan {
   int first;  // the context's first unit
   int per;    // tiles per split

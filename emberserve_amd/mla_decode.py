@@ -15,7 +15,10 @@ fp32. CPU tensors take the eager form of mla_attention_absorbed with identity W
 (attn/mla_torch.py:33-53), the definition the reference tests compare the kernel with.
 
 The split count comes from shapes only, so a captured HIP graph replays exactly what was
-captured; the split-K scratch is cached per shape for the same reason.
+captured; the split-K scratch is cached per shape for the same reason. Where the splits cut a
+batch does not: from 4 splits of 512 keys of table width, the kernel sizes them from all of a
+batch's context lengths, so a sequence's rounding (not its numerics) can differ beside other
+sequences. With num_splits below 4 each sequence is cut by its own length.
 """
 
 from __future__ import annotations
