@@ -370,6 +370,26 @@ def test_decode_shapes_take_turns_on_one_workspace(monkeypatch):
     assert len(pd._SCRATCH._bufs) == 1 and _lib.read_errors() == 0
 
 
+@pytest.mark.parametrize("batch,hq,hkv,d,splits", [(9, 32, 8, 128, 3), (13, 40, 2, 128, 5), (7, 6, 3, 64, 1), (1, 8, 1, 64, 4)])
+def test_decode_shared_prefix_blocks(batch, hq, hkv, d, splits):
+    """Sequences whose tables begin with the same blocks give the bits of tables over copies of those
+    blocks; batches whose (split, sequence, KV head) count is no multiple of the XCDs."""
+    prefix = 12
+    ctx = [16 * prefix + 1 + 37 * i for i in range(batch)]
+    q, kc, vc, bt, cl = _to_dev(*gen.decode_inputs(ctx, hq, hkv, d, 16, torch.bfloat16, seed=40))
+    copies = bt[1:, :prefix].long()
+    kc[copies], vc[copies] = kc[bt[0, :prefix].long()], vc[bt[0, :prefix].long()]
+    shared = bt.clone()
+    shared[:, :prefix] = bt[0, :prefix]
+    _say(f"shared prefix B={batch} {hq}q/{hkv}kv x{d} splits={splits}")
+    want = paged_attention_decode(q, kc, vc, bt, cl, d ** -0.5, num_splits=splits)
+    assert torch.equal(paged_attention_decode(q, kc, vc, shared, cl, d ** -0.5, num_splits=splits), want)
+    o = ref.paged_decode(q.float().cpu(), kc.cpu(), vc.cpu(), bt.cpu(), cl.cpu(), d ** -0.5)
+    mass = ref.paged_decode_prob_mass(q.float().cpu(), kc.cpu(), vc.cpu(), bt.cpu(), cl.cpu(), d ** -0.5)
+    u = U[torch.bfloat16]
+    assert bool(((want.float().cpu() - o).abs() <= 1.1 * u * (mass + o.abs()) + 1e-4 * mass + 1e-6).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_decode_entry_points_keep_their_counters_apart(dtype):
     """Over a workspace larger than the call's need, ember_paged_decode's counters follow its
