@@ -235,14 +235,20 @@ def gate_up_silu_gemm_packed(x: Tensor, packed: PackedGateUp, *, column_tile: in
 
 def packed_gemm_default(tokens: int, hidden: int, inter: int, device: torch.device) -> bool:
     """Whether the packed GEMM runs by default above PACKED_FUSED_TOKENS when the unpacked
-    weight is there too: while its tiles fit the CUs in one round, and at any size for short
-    rows, where the projection's round trip through memory is long against its product.
-    Measured (bf16, us, packed GEMM | hipBLASLt + silu_and_mul): Qwen3-8B 64 tokens 41 | 45,
-    128: 46 | 50, 160: 51 | 55, 200: 60 | 63, 256: 63 | 65, 300: 70 | 76, 512: 90 | 91, but 2048: 317 | 301;
-    Qwen2.5-7B 64: 51 | 62, 128: 56 | 70, 256: 80 | 82, but 600: 188 | 172; Qwen2.5-0.5B (H 896)
-    100: 9.3 | 13, 1024: 27 | 37, 8192: 161 | 199."""
-    return _gemm_takes(hidden, inter) and (hidden <= 1024
-                                           or -(-tokens // 256) * -(-inter // 128) <= num_sms(device))
+    weight is there too: for short rows, where the projection's round trip through memory is long
+    against its product, and else while its largest tiles fit the CUs in one round and its smallest
+    would fill 5/8 of them. Measured (bf16, us, packed GEMM | hipBLASLt + silu_and_mul, replayed):
+    Qwen3-8B 64 tokens 42 | 52, 128: 46 | 50, 200: 60 | 63, 512: 90 | 91, but 2000 1.10 times as long;
+    Qwen2.5-7B 64: 56 | 70, but 600 1.04 times; Qwen2.5-0.5B (H 896) 100: 9.3 | 13, 8192: 161 | 199.
+    Too few tiles (H x I, tokens): 4096 x 1536, 40: 28 | 16, 4096 x 4096, 64: 1.38 times, 7168 x 2048,
+    40: 1.95 times, but 2048 x 5632, 64: 0.98 (176 tiles), 4096 x 4096, 160: 0.95 (256), 1024 x 256,
+    40: 1.13 and 1024 x 768: 0.88."""
+    if not _gemm_takes(hidden, inter):
+        return False
+    if hidden <= min(1024, 2 * inter):
+        return True
+    cus = num_sms(device)
+    return -(-tokens // 256) * -(-inter // 128) <= cus and 8 * -(-tokens // 128) * -(-inter // 32) >= 5 * cus
 
 
 def _gemm_takes(hidden: int, inter: int) -> bool:

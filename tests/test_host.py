@@ -343,7 +343,23 @@ def test_gate_up_silu_sizes_past_the_packed_gemm_keep_their_kernels(monkeypatch,
     x = torch.empty(48, hidden, dtype=torch.bfloat16, device="meta")
     assert mod.gate_up_silu(x, None, packed=packed) == ("gemm" if gemm else "decode")
     assert mod.gate_up_silu(x[:32], None, packed=packed) == "decode"
-    assert mod.packed_gemm_default(48, hidden, inter, torch.device("cpu")) == gemm
+    assert mod._gemm_takes(hidden, inter) == gemm
+    if not gemm:
+        assert not mod.packed_gemm_default(48, hidden, inter, torch.device("cpu"))
+
+
+def test_packed_gemm_default_rule(monkeypatch):
+    """One round of the largest tiles, 5/8 of the CUs filled by the smallest; short rows at any size
+    unless the columns are fewer than half of them."""
+    from emberserve_amd import gate_up_silu as mod
+    monkeypatch.setattr(mod, "num_sms", lambda device: 256)
+    rule = lambda t, h, i: mod.packed_gemm_default(t, h, i, torch.device("cpu"))  # noqa: E731
+    assert [rule(t, 4096, 12288) for t in (33, 512, 513)] == [True, True, False]
+    assert [rule(t, 896, 4864) for t in (33, 8192)] == [True, True]
+    assert [rule(t, 4096, 1536) for t in (40, 384, 385)] == [False, False, True]
+    assert [rule(t, 4096, 4096) for t in (64, 128, 129)] == [False, False, True]
+    assert [rule(64, h, i) for h, i in ((2048, 5632), (5120, 5120), (2048, 5088), (7168, 2048))] == [True, True, False, False]
+    assert [rule(40, 1024, i) for i in (256, 512, 768)] == [False, True, True]
 
 
 def test_gate_up_silu_workspace_plan():
