@@ -44,6 +44,7 @@ MAX_TOKENS = 64           # the kernels' limit
 PACKED_MAX_TOKENS = 64
 FUSED_TOKENS = 16         # default dispatch, row kernel: the kernel up to here, the pair above
 PACKED_FUSED_TOKENS = 32  # default dispatch over a packed weight
+PACKED_WIDE_TOKENS = 48   # ... over the packed copy alone, packed for more than 3/4 of the CUs
 # Prefill sizes (gate_up_silu_gemm): 256-token tiles of 64, 96 or 128 gate (and as many up)
 # columns. A workgroup's time follows the bytes it streams from L2 into LDS (all 256 x rows
 # plus its 2·columns weight rows, at ~40-45 GB/s per CU), so the call takes about
@@ -262,16 +263,22 @@ def gate_up_silu(x: Tensor, weight: Tensor | None, *, num_workgroups: int | None
     (`pack_gate_up_weight(weight)`), the fused kernel reads the packed copy instead. With
     `packed` and weight None (a model that dropped the unpacked weight) every size runs on
     the packed copy: the decode kernel up to PACKED_FUSED_TOKENS tokens (PACKED_MAX_TOKENS when
-    num_workgroups, which is the decode kernel's, is given), the packed prefill GEMM above
-    (33-64 tokens, us, decode kernel | GEMM: Qwen3-8B 39-42 | 40-41, Qwen2.5-7B 63-68 | 50,
-    Qwen2.5-0.5B 12 | 9)."""
+    num_workgroups, which is the decode kernel's, is given, PACKED_WIDE_TOKENS when its grid is wide
+    enough to stream the weights as fast as the GEMM's does), the packed prefill GEMM above. 40 tokens,
+    us, workgroups, decode kernel | GEMM: H 4096 x I 14336 224, 42 | 46.5, 5120 x 13824 216, 54 | 60,
+    1024 x 16384 256, 15.6 | 16.7, Qwen3-8B 192, 41 | 41, 4096 x 11008 172, 40 | 39.5, Qwen2.5-7B 148,
+    70 | 54, 2048 x 8192 128, 22 | 19, Qwen2.5-0.5B 76, 12 | 10; at 64 tokens 46 | 48, 59 | 59, 17.3 |
+    17.6, 45 | 42."""
     if weight is None:
         if packed is None:
             raise ValueError("gate_up_silu: weight None needs the packed weight")
         if fused is False:
             raise ValueError("gate_up_silu: the unfused pair needs the unpacked weight")
-        gemm = num_workgroups is None and _gemm_takes(packed.hidden, packed.inter)
-        limit = PACKED_FUSED_TOKENS if gemm else PACKED_MAX_TOKENS
+        if num_workgroups is not None or not _gemm_takes(packed.hidden, packed.inter):
+            limit = PACKED_MAX_TOKENS
+        else:
+            wide = 4 * packed.num_workgroups > 3 * num_sms(packed.device)
+            limit = PACKED_WIDE_TOKENS if wide else PACKED_FUSED_TOKENS
         if x.reshape(-1, packed.hidden).shape[0] > limit:
             return gate_up_silu_gemm_packed(x, packed)
         return _packed_decode(x, packed, num_workgroups)

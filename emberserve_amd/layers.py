@@ -53,7 +53,7 @@ class SwiGLUMLP(nn.Module):
     modified in place, and the forward then reads the weight itself.
     `pack_weights(keep_weight=False)` instead replaces the weight by its packed copy: the
     module then holds one copy of the gate_up weight (gate_up_proj.weight becomes an empty
-    tensor) and every batch runs on the packed copy, the decode kernel up to 32 tokens and
+    tensor) and every batch runs on the packed copy, the decode kernel up to 32 or 48 tokens and
     the packed prefill GEMM above. Load checkpoints before dropping the weight."""
 
     def __init__(self, hidden_size: int, intermediate_size: int) -> None:

@@ -348,6 +348,18 @@ def test_gate_up_silu_sizes_past_the_packed_gemm_keep_their_kernels(monkeypatch,
         assert not mod.packed_gemm_default(48, hidden, inter, torch.device("cpu"))
 
 
+@pytest.mark.parametrize("workgroups,limit", [(148, 32), (192, 32), (193, 48), (256, 48)])
+def test_gate_up_silu_packed_alone_limits(monkeypatch, workgroups, limit):
+    """Over the packed copy alone, a grid over 3/4 of the CUs keeps the decode kernel up to 48 tokens."""
+    from emberserve_amd import gate_up_silu as mod
+    monkeypatch.setattr(mod, "num_sms", lambda device: 256)
+    monkeypatch.setattr(mod, "gate_up_silu_gemm_packed", lambda x, packed: "gemm")
+    monkeypatch.setattr(mod, "_packed_decode", lambda x, packed, n: "decode")
+    packed = mod.PackedGateUp(torch.empty(0, dtype=torch.bfloat16), 256, 256, workgroups)
+    got = [mod.gate_up_silu(torch.empty(t, 256, dtype=torch.bfloat16), None, packed=packed) for t in range(1, 66)]
+    assert got == ["decode"] * limit + ["gemm"] * (65 - limit)
+
+
 def test_packed_gemm_default_rule(monkeypatch):
     """One round of the largest tiles, 5/8 of the CUs filled by the smallest; short rows at any size
     unless the columns are fewer than half of them."""
